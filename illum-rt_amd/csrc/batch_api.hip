@@ -95,10 +95,17 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
         rt::scene_desc fmt{};
         fmt.bvh = bvh;
         fmt.tri = tri;
-        HIP_TRY(hiprt_detail::attach_spill(st, s, fmt, any != 0, true, need[g.first], cfg, opts ? opts->spill_limit : 0));
+        // few rays in all: several lanes per ray (no spill column, no counters)
+        const bool own_kernel = opts && (opts->blocks > 0 || opts->spill_limit > 0);
+        const int lanes = own_kernel ? 0 : rt::dev::group_lanes(bvh, need[g.first], (uint32_t)totals[g.first]);
+        if (!lanes) HIP_TRY(hiprt_detail::attach_spill(st, s, fmt, any != 0, true, need[g.first], cfg, opts ? opts->spill_limit : 0));
         auto *dst = reinterpret_cast<rt::dev::batch_desc *>(static_cast<char *>(table.p) + off);
         HIP_TRY(hipMemcpy(dst, g.second.data(), g.second.size() * sizeof(rt::dev::batch_desc), hipMemcpyHostToDevice));
-        HIP_TRY(rt::dev::launch_trace_batch(dst, (uint32_t)g.second.size(), (uint32_t)totals[g.first], tri, bvh,
+        if (lanes)
+            HIP_TRY(rt::dev::launch_trace_group_batch(dst, (uint32_t)g.second.size(), (uint32_t)totals[g.first], tri,
+                                                      any != 0, lanes, need[g.first], s));
+        else
+            HIP_TRY(rt::dev::launch_trace_batch(dst, (uint32_t)g.second.size(), (uint32_t)totals[g.first], tri, bvh,
                                             any != 0, st->counter.as<uint32_t>(), cfg, s));
         off += g.second.size() * sizeof(rt::dev::batch_desc);
     }

@@ -817,6 +817,17 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     if (tracer == HIPRT_TRACER_WHILE_WHILE) {
         if (need > rt::dev::kPlainStackCap - 1)
             return fail(HIPRT_ERR_UNSUPPORTED, "BVH deeper than the traversal stack (" + std::to_string(need) + " entries)");
+    }
+    // Small batches: several lanes per ray, whichever tracer was asked for
+    // (its hits are the plain tracer's, which every tracer returns up to
+    // ties).  A caller that counts fetches, sets the grid or bounds the spill
+    // column gets the kernel those belong to.
+    const bool own_kernel = opts && (opts->d_fetch_stats || opts->blocks > 0 || opts->spill_limit > 0);
+    if (int lanes = own_kernel ? 0 : rt::dev::group_lanes(desc.bvh, need, n)) {
+        HIP_TRY(rt::dev::launch_trace_group(desc, r, h, occluded, n, nullptr, any, lanes, need, s));
+        return ok();
+    }
+    if (tracer == HIPRT_TRACER_WHILE_WHILE) {
         HIP_TRY(rt::dev::launch_trace_plain(desc, r, h, occluded, n, any, s,
                                             opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats)
                                                  : nullptr));

@@ -111,6 +111,30 @@ hipError_t launch_trace_batch(const batch_desc *d_table, uint32_t n_desc, uint32
 hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg &cfg, int *blocks,
                            bool multi = false);
 
+// Group trace (trace_group.hip): `lanes` lanes per ray, for batches too small
+// to fill the chip with one ray per lane.  group_lanes: 16 up to kGroupRays16
+// rays, 8 up to kGroupRays8, else 0 (and for 4-wide or very deep trees):
+// the persistent and plain kernels serve those.
+//   16 -> 8: the two met at 65k-77k rays on the hall (91 / 95 us at 37k, 147 /
+//   147 at 77k) and at 40k on the 8,192-triangle scene.
+//   8 -> 0: 640 x 480 (307k) rays took 433 / 410 us (camera / bounce) against
+//   535 / 640 with the dynamic tracer and 813 / 1034 with the plain one,
+//   1280 x 720 (922k) 1069 / 1088 against 728 / 1012 and 1108 / 1801.
+constexpr int kGroupStackNeed = 64;
+constexpr uint32_t kGroupRays16 = 1u << 16;
+constexpr uint32_t kGroupRays8 = 1u << 19;
+int group_lanes(int bvh, int need, uint32_t n);
+// The hits (or occlusion) of n rays (of *count_ptr, when given, at most n) of
+// a binary tree with stack need `need` <= kGroupStackNeed; no device memory
+// besides the arguments.  Rays, hits and gather as launch_trace_persistent;
+// the results are the plain kernel's, bit for bit.
+hipError_t launch_trace_group(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,
+                              uint32_t n, const uint32_t *count_ptr, bool any, int lanes, int need, hipStream_t s,
+                              ray_gather gather = ray_gather{});
+// The same over a descriptor table, as launch_trace_batch.
+hipError_t launch_trace_group_batch(const batch_desc *d_table, uint32_t n_desc, uint32_t total, int tri, bool any,
+                                    int lanes, int need, hipStream_t s);
+
 // Fills `n` uint32 words with `value` (used instead of hipMemsetAsync so the
 // clearing can be captured into graphs).
 hipError_t launch_fill_u32(uint32_t *p, uint32_t value, uint32_t n, hipStream_t stream);

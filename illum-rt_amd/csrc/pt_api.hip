@@ -100,6 +100,7 @@ struct hiprt_pt_s {
     bool batched = false;
     bool jitter = true;   // camera rays through a random point of the pixel (else its centre)
     rt::dev::persistent_cfg pcfg{};
+    int group = 0;        // lanes per ray of the group trace; 0: the persistent or plain kernel traces
     // refill threshold of levels 0 and 1 with a pixel's samples in flight:
     // queued pixel-major, a wavefront holds one pixel's camera rays (and,
     // sorted, rays leaving nearby points), and refilling it early mixes in
@@ -151,6 +152,17 @@ struct hiprt_pt_s {
                                            sort_counts.as<uint32_t>(), sort_totals.as<uint32_t>()};
     }
 
+    // One trace launch of the batched schedule: the rays of `in` (or the
+    // records of g), *count of them.  The counting variant (cfg.stats) and a
+    // caller's own grid use the persistent kernel.
+    hipError_t trace(const rt::ray_soa &in, const uint32_t *count, const rt::dev::persistent_cfg &cfg, hipStream_t s,
+                     const rt::dev::ray_gather &g = rt::dev::ray_gather{}) {
+        const rt::scene_desc d = hiprt_detail::desc_for(sc, alpha);
+        if (group && !cfg.stats)
+            return rt::dev::launch_trace_group(d, in, h, nullptr, n, count, false, group, sc->stack_need, s, g);
+        return rt::dev::launch_trace_persistent(d, in, h, nullptr, n, count, work.as<uint32_t>(), false, cfg, s, g);
+    }
+
     // kRegenChunk regeneration iterations: trace the queue in record buffer
     // a, shade it into buffer b (continued paths and regenerated camera
     // rays), sort b's keys.
@@ -165,8 +177,7 @@ struct hiprt_pt_s {
             g.perm = sorted ? perm.as<const uint32_t>() : nullptr;
             g.stride = kRayRecord;
             g.fixed_t = 1;
-            hipError_t e = launch_trace_persistent(hiprt_detail::desc_for(sc, alpha), rt::ray_soa{}, h, nullptr, n,
-                                                   q + a, work.as<uint32_t>(), false, pcfg, s, g);
+            hipError_t e = trace(rt::ray_soa{}, q + a, pcfg, s, g);
             if (e == hipSuccess) e = launch_fill_u32(q + b, 0u, 1u, s);
             if (e == hipSuccess)
                 e = launch_shade_regen(ps(), pp, rp, rec[a].as<const float4>(), g.perm, h, rec[b].as<float4>(),
@@ -245,8 +256,12 @@ struct hiprt_pt_s {
             }
             unsigned long long *lstats = stats ? stats + 2 * L : nullptr;
             if (!batched) {
-                e = launch_trace_plain(hiprt_detail::desc_for(sc, alpha), rays[0].out.as_in(), h, nullptr, n, false, s,
-                                       lstats);
+                if (group && !lstats)
+                    e = launch_trace_group(hiprt_detail::desc_for(sc, alpha), rays[0].out.as_in(), h, nullptr, n,
+                                           nullptr, false, group, sc->stack_need, s);
+                else
+                    e = launch_trace_plain(hiprt_detail::desc_for(sc, alpha), rays[0].out.as_in(), h, nullptr, n,
+                                           false, s, lstats);
                 if (e != hipSuccess) return e;
                 if (ev) {
                     e = hipEventRecord(ev[2 * L + 1], s);
@@ -260,9 +275,7 @@ struct hiprt_pt_s {
                 if (pp.px_samples > 1 && L <= 1) cfg.refill_thr = refill_coherent;
                 if (!sorted) {
                     const ray_planes &in = rays[L & 1], &outq = rays[(L + 1) & 1];
-                    e = launch_trace_persistent(hiprt_detail::desc_for(sc, alpha), in.out.as_in(), h, nullptr, n,
-                                                cnt + L,
-                                                work.as<uint32_t>(), false, cfg, s);
+                    e = trace(in.out.as_in(), cnt + L, cfg, s);
                     if (e != hipSuccess) return e;
                     if (ev) {
                         e = hipEventRecord(ev[2 * L + 1], s);
@@ -281,9 +294,7 @@ struct hiprt_pt_s {
                     g.aos = in_rec;
                     g.perm = pm;
                     g.stride = kRayRecord;
-                    e = launch_trace_persistent(hiprt_detail::desc_for(sc, alpha), rays[0].out.as_in(), h, nullptr,
-                                                n, cnt + L,
-                                                work.as<uint32_t>(), false, cfg, s, g);
+                    e = trace(rays[0].out.as_in(), cnt + L, cfg, s, g);
                     if (e != hipSuccess) return e;
                     if (ev) {
                         e = hipEventRecord(ev[2 * L + 1], s);
@@ -684,6 +695,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
     HIP_TRY(hipMemset(p->totals.p, 0, 8ull * (p->pp.max_depth + 1)));
     HIP_TRY(p->frame_seed.alloc(8ull * samples));
     HIP_TRY(p->work.alloc(rt::dev::kCounterBytes));
+    if (params->blocks <= 0) p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n);
     p->pcfg.speculative = p->tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
     p->pcfg.refill = p->tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
     p->pcfg.refill_thr = params->refill_threshold > 0 ? std::min(params->refill_threshold, 64) : 40;
