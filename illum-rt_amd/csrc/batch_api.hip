@@ -97,7 +97,8 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
         fmt.tri = tri;
         // few rays in all: several lanes per ray (no spill column, no counters)
         const bool own_kernel = opts && (opts->blocks > 0 || opts->spill_limit > 0);
-        const int lanes = own_kernel ? 0 : rt::dev::group_lanes(bvh, need[g.first], (uint32_t)totals[g.first]);
+        const uint32_t rays8 = !any && cfg.speculative ? rt::dev::kGroupRays8Spec : rt::dev::kGroupRays8;
+        const int lanes = own_kernel ? 0 : rt::dev::group_lanes(bvh, need[g.first], (uint32_t)totals[g.first], rays8);
         if (!lanes) HIP_TRY(hiprt_detail::attach_spill(st, s, fmt, any != 0, true, need[g.first], cfg, opts ? opts->spill_limit : 0));
         auto *dst = reinterpret_cast<rt::dev::batch_desc *>(static_cast<char *>(table.p) + off);
         HIP_TRY(hipMemcpy(dst, g.second.data(), g.second.size() * sizeof(rt::dev::batch_desc), hipMemcpyHostToDevice));

@@ -823,12 +823,14 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     // ties).  A caller that counts fetches, sets the grid or bounds the spill
     // column gets the kernel those belong to.
     const bool own_kernel = opts && (opts->d_fetch_stats || opts->blocks > 0 || opts->spill_limit > 0);
-    if (int lanes = own_kernel ? 0 : rt::dev::group_lanes(desc.bvh, need, n)) {
+    const bool postpones = !any && tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
+    const uint32_t rays8 = postpones ? rt::dev::kGroupRays8Spec : rt::dev::kGroupRays8;
+    if (int lanes = own_kernel ? 0 : rt::dev::group_lanes(desc.bvh, need, n, rays8)) {
         HIP_TRY(rt::dev::launch_trace_group(desc, r, h, occluded, n, nullptr, any, lanes, need, s));
         return ok();
     }
     if (tracer == HIPRT_TRACER_WHILE_WHILE) {
-        HIP_TRY(rt::dev::launch_trace_plain(desc, r, h, occluded, n, any, s,
+        HIP_TRY(rt::dev::launch_trace_plain(desc, r, h, occluded, n, any, need, s,
                                             opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats)
                                                  : nullptr));
         return ok();

@@ -11,8 +11,8 @@
 namespace rt {
 namespace dev {
 
-// Private-memory stack of the plain kernels; the host refuses BVHs deeper
-// than kPlainStackCap - 1 inner levels for them.
+// The plain kernels hold their stack in LDS (256 bytes a block and entry);
+// the host refuses BVHs that need kPlainStackCap or more entries for them.
 constexpr int kPlainStackCap = 64;
 
 // Persistent kernels, stack configuration 0: per-lane stack of kRegStack
@@ -54,10 +54,11 @@ struct batch_desc {
     uint32_t first, n;
 };
 
-// With `stats` non-null the counting variant runs and adds the number of inner
-// nodes fetched to stats[0] and of triangle records tested to stats[1].
+// `need`: the tree's stack need, below kPlainStackCap.  With `stats` non-null
+// the counting variant runs and adds the number of inner nodes fetched to stats[0] and of triangle records tested to stats[1].
 hipError_t launch_trace_plain(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,
-                              uint32_t n, bool any, hipStream_t stream, unsigned long long *stats = nullptr);
+                              uint32_t n, bool any, int need, hipStream_t stream,
+                              unsigned long long *stats = nullptr);
 
 // Rays of a single-scene persistent launch read from records of `stride`
 // float4 (at least two) that begin (ox, oy, oz, tmin | dx, dy, dz, tmax)
@@ -113,17 +114,24 @@ hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg 
 
 // Group trace (trace_group.hip): `lanes` lanes per ray, for batches too small
 // to fill the chip with one ray per lane.  group_lanes: 16 up to kGroupRays16
-// rays, 8 up to kGroupRays8, else 0 (and for 4-wide or very deep trees):
-// the persistent and plain kernels serve those.
-//   16 -> 8: the two met at 65k-77k rays on the hall (91 / 95 us at 37k, 147 /
-//   147 at 77k) and at 40k on the 8,192-triangle scene.
-//   8 -> 0: 640 x 480 (307k) rays took 433 / 410 us (camera / bounce) against
-//   535 / 640 with the dynamic tracer and 813 / 1034 with the plain one,
-//   1280 x 720 (922k) 1069 / 1088 against 728 / 1012 and 1108 / 1801.
+// rays, 8 up to kGroupRays8 (kGroupRays8Spec for the closest hits of the
+// postponing tracers), else 0, and 0 for 4-wide or very deep trees: the plain
+// and persistent kernels serve those.  Hall, us, camera / bounce rays:
+//   16 -> 8: 320 x 240 (77k) 124 / 131 against 129 / 139, but 53 / 41 against
+//   43 / 44 in the 8,192-triangle scene.
+//   8 -> 0: 800 x 600 (480k) 496 / 526, plain 631 / 851, dynamic 699 / 855;
+//   1281 x 719 (921k) 832 / 910, plain 787 / 1220, dynamic 723 / 1027 (any
+//   hit 730 / 781, plain 784 / 1191, dynamic 805 / 1191);
+//   1920 x 1080 (2.07M) 1734 / 1912, plain 1250 / 2262, dynamic 1118 / 1678.
+// A path tracer's later levels hold ever fewer of its slots: kGroupSlots8.
+// Whole frames: 1280 x 720 (921k) 4.19 ms, dynamic 4.83; 320 x 240 x 16
+// samples (1.23M) 5.41 against 5.82.
 constexpr int kGroupStackNeed = 64;
 constexpr uint32_t kGroupRays16 = 1u << 16;
-constexpr uint32_t kGroupRays8 = 1u << 19;
-int group_lanes(int bvh, int need, uint32_t n);
+constexpr uint32_t kGroupRays8 = 1u << 20;
+constexpr uint32_t kGroupRays8Spec = 5u << 17;
+constexpr uint32_t kGroupSlots8 = 5u << 18;
+int group_lanes(int bvh, int need, uint32_t n, uint32_t rays8);
 // The hits (or occlusion) of n rays (of *count_ptr, when given, at most n) of
 // a binary tree with stack need `need` <= kGroupStackNeed; no device memory
 // besides the arguments.  Rays, hits and gather as launch_trace_persistent;

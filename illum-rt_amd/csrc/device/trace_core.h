@@ -21,6 +21,18 @@
 namespace rt {
 namespace dev {
 
+// Work index of block b of nb.  Workgroup b runs on XCD b mod 8: of every 8 *
+// seg consecutive indices each XCD takes seg neighbours, so rays of one
+// neighbourhood share an L2, and every XCD gets a share of each part of the
+// batch (one contiguous eighth per XCD left the XCDs with the cheap parts of
+// a camera image idle: 640 x 480 rays of the hall 433 us, with this 352 us).
+// A bijection on [0, nb): the last, incomplete span keeps its order.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb, uint32_t seg) {
+    const uint32_t span = 8u * seg, s0 = b / span * span;
+    if (nb - s0 < span) return b;
+    return s0 + (b & 7u) * seg + ((b - s0) >> 3);
+}
+
 struct dray {
     float ox, oy, oz, tmin, dx, dy, dz, tmax;
     float ix, iy, iz;   // 1/d, computed as ray::ray does (libgi/rt.h:28)
@@ -238,12 +250,16 @@ __device__ __forceinline__ uint32_t slot_tri_id(const scene_desc &sc, uint32_t s
     return sc.slot_ids[slot];
 }
 
+// A while-while wavefront leaves its node loop once at most this many lanes
+// still descend: the lanes that hold a leaf do not wait for the last few.
+// Each lane's own order is unchanged.  (Measured beside k_trace_plain.)
+constexpr int kNodeLanes = 8;
+
 // Result of one ray.
 struct dhit {
     float t, u, v;
     uint32_t slot;
     bool found;
-    bool over;   // the traversal dropped a stack entry: the result is not known
 };
 
 __device__ __forceinline__ void store_hit(const hit_soa &h, uint32_t i, float t, float u, float v, uint32_t id) {

@@ -35,10 +35,10 @@
 // node step, 110 a leaf step; of 8 lanes 5.0 hold an inner node on camera
 // rays and 4.0 on bounce rays; 29 and 33 node steps, 11 and 15 leaf steps per
 // wavefront of 8 rays), the latency of the dependent node fetches below that.
-// Measured, closest hit, hall, one ray per lane (plain kernel) against this
-// one: 64 x 48 camera rays 670 -> 41 us (K = 16), 320 x 240 743 -> 147 us,
-// 640 x 480 813 -> 433 us, 1280 x 720 1108 -> 1069 us (K = 8); bounce rays
-// 581 -> 38, 787 -> 136, 1034 -> 410, 1801 -> 1088 us.  K = 4 was slower than
+// Measured, closest hit, hall, one ray per lane (plain kernel before its vote
+// and LDS stack) against this one: 64 x 48 camera rays 670 -> 38 us (K = 16),
+// 320 x 240 743 -> 124 us, 640 x 480 813 -> 352 us, 1281 x 719 1108 -> 832 us
+// (K = 8); bounce rays 581 -> 35, 787 -> 131, 1034 -> 381, 1801 -> 910 us.  K = 4 was slower than
 // 8 at the sizes this kernel serves (640 x 480: 554 against 468 us), fetching
 // the nodes before the leaf step the same within 2% at fewer waves, refilling
 // idle groups from a work counter slower (1280 x 720: 1290 against 1069 us: a
@@ -133,19 +133,18 @@ __device__ __forceinline__ bool box_min3(float xlo, float xhi, float ylo, float 
 } // namespace
 
 template <int K, int TRI, bool ANY, bool MULTI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MULTI ? 7 : 8)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MULTI ? 7 : 8)))
 void k_trace_group(group_args a) {
     extern __shared__ group_entry lds_entries[];
     const uint32_t n = a.count_ptr ? min(*a.count_ptr, a.n) : a.n;
-    const uint32_t lane = threadIdx.x & 63u, gl = lane & (K - 1), shift = lane & ~(uint32_t)(K - 1);
-    constexpr uint32_t kRays = 256u / K;   // rays per block
+    const uint32_t lane = threadIdx.x, gl = lane & (K - 1), shift = lane & ~(uint32_t)(K - 1);
+    constexpr uint32_t kRays = 64u / K;   // rays per block
     const uint32_t low = (1u << gl) - 1u;
     group_entry *st = lds_entries + (threadIdx.x / K) * a.cap;
 
-    // XCD x takes the x-th eighth of the blocks
-    const uint32_t nb = (n + kRays - 1) / kRays, x = blockIdx.x & 7u, per = nb >> 3, extra = nb & 7u;
+    const uint32_t nb = (n + kRays - 1) / kRays;
     if (blockIdx.x >= nb) return;
-    const uint32_t idx = (x * per + min(x, extra) + (blockIdx.x >> 3)) * kRays + threadIdx.x / K;
+    const uint32_t idx = xcd_block(blockIdx.x, nb, 16u) * kRays + threadIdx.x / K;
     const bool has = idx < n;
 
     uint32_t ray_id = 0, desc = 0;
@@ -361,10 +360,10 @@ namespace {
 
 template <int K, int TRI, bool ANY, bool MULTI>
 hipError_t launch_k(const group_args &a, hipStream_t s) {
-    constexpr uint32_t kRays = 256u / K;
+    constexpr uint32_t kRays = 64u / K;
     const uint32_t blocks = (a.n + kRays - 1) / kRays;
     const size_t lds = kRays * a.cap * sizeof(group_entry);
-    hipLaunchKernelGGL((k_trace_group<K, TRI, ANY, MULTI>), dim3(blocks), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((k_trace_group<K, TRI, ANY, MULTI>), dim3(blocks), dim3(64), lds, s, a);
     return hipGetLastError();
 }
 
@@ -377,8 +376,8 @@ hipError_t dispatch(int tri, bool any, const group_args &a, hipStream_t s) {
 
 template <bool MULTI>
 hipError_t dispatch_lanes(int lanes, int tri, bool any, int need, group_args &a, hipStream_t s) {
-    // 8 lanes: 32 rays a block, 64 entries for the hall's need of 22, so 8
-    // blocks share a CU's LDS
+    // one wavefront a block, so that its LDS is free when its slowest ray
+    // ends; 8 lanes and the hall's stack need of 22: 72 entries a ray, 4.6 KB
     a.soft = lanes == 8 ? 40u : 64u;
     a.cap = a.soft + (uint32_t)need + 2u;
     // groups whose lists are equally long read different LDS banks
@@ -389,9 +388,9 @@ hipError_t dispatch_lanes(int lanes, int tri, bool any, int need, group_args &a,
 
 } // namespace
 
-int group_lanes(int bvh, int need, uint32_t n) {
+int group_lanes(int bvh, int need, uint32_t n, uint32_t rays8) {
     if (bvh != BVH2 || need > kGroupStackNeed) return 0;
-    return n <= kGroupRays16 ? 16 : (n <= kGroupRays8 ? 8 : 0);
+    return n <= kGroupRays16 ? 16 : (n <= rays8 ? 8 : 0);
 }
 
 hipError_t launch_trace_group(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,

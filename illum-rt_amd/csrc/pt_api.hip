@@ -261,7 +261,7 @@ struct hiprt_pt_s {
                                            nullptr, false, group, sc->stack_need, s);
                 else
                     e = launch_trace_plain(hiprt_detail::desc_for(sc, alpha), rays[0].out.as_in(), h, nullptr, n,
-                                           false, s, lstats);
+                                           false, sc->stack_need, s, lstats);
                 if (e != hipSuccess) return e;
                 if (ev) {
                     e = hipEventRecord(ev[2 * L + 1], s);
@@ -695,7 +695,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
     HIP_TRY(hipMemset(p->totals.p, 0, 8ull * (p->pp.max_depth + 1)));
     HIP_TRY(p->frame_seed.alloc(8ull * samples));
     HIP_TRY(p->work.alloc(rt::dev::kCounterBytes));
-    if (params->blocks <= 0) p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n);
+    if (params->blocks <= 0) p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n, rt::dev::kGroupSlots8);
     p->pcfg.speculative = p->tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
     p->pcfg.refill = p->tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
     p->pcfg.refill_thr = params->refill_threshold > 0 ? std::min(params->refill_threshold, 64) : 40;

@@ -12,6 +12,7 @@ import pytest
 import hiprt
 import oracle_py as orc
 from parity import bit_exact, classify, uniform_sphere_rays
+from test_gpu_spill import nested_rays, nested_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -56,10 +57,10 @@ def test_batch_sizes(torch_cuda, hip_ctx, soup, n):
     _check(torch_cuda, hip_ctx, *soup, uniform_sphere_rays(n, n))
 
 
-@pytest.mark.parametrize("n", [524287, 524288, 524289])
+@pytest.mark.parametrize("n", [655360, 655361, 1048576, 1048577])
 def test_switch_to_one_ray_per_lane(torch_cuda, hip_ctx, soup, n):
     print(f"case: {n} rays, the largest group batch", flush=True)
-    _check(torch_cuda, hip_ctx, *soup, uniform_sphere_rays(n, 3), tracers=("while-while",))
+    _check(torch_cuda, hip_ctx, *soup, uniform_sphere_rays(n, 3), tracers=("while-while", "persistent-while-while"))
 
 
 @pytest.mark.parametrize("max_tris", [1, 4, 5, 9, 17, 32])
@@ -154,3 +155,21 @@ def test_alpha_and_batch(torch_cuda, hip_ctx):
         got = tuple(h[k].cpu().numpy() for k in ("t", "u", "v")) + (h["id"].cpu().numpy().view(np.uint32),)
         assert bit_exact(got, want)
         ds.close()
+
+
+def test_deep_tree(torch_cuda, hip_ctx):
+    """The nested triangles' 38-level tree: the group kernel's list, and the
+    plain kernel's LDS stack (its counting variant)."""
+    torch = torch_cuda
+    pos, idx = nested_scene()
+    sc = hiprt.HostScene.from_arrays(pos, idx)
+    bvh = hiprt.Bvh(sc, max_tris=1)
+    ds = hiprt.DeviceScene(hip_ctx, sc, bvh)
+    assert 24 < ds.stack_need < 64, ds.stack_need
+    for n in (4000, 70000):
+        rays = nested_rays(n, n)
+        want = orc.trace_closest(pos, idx, bvh.nodes, bvh.root, bvh.index, rays)
+        assert bit_exact(_closest(torch, ds, rays), want)
+        stats = torch.zeros(2, dtype=torch.int64, device="cuda")
+        assert bit_exact(_closest(torch, ds, rays, fetch_stats=stats), want)
+    ds.close()
