@@ -480,6 +480,8 @@ void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
     s->desc.tri = h.tri_kind;
     s->desc.depth = (int32_t)h.depth;
     s->stack_need = (int)stack_need;
+    s->n_nodes = (uint32_t)(h.bvh_kind == rt::BVH2 ? h.nodes2.size() : h.nodes4.size());
+    s->n_slots = (uint32_t)h.tris.size();
     {
         // box bounds of absent 4-wide children are +-inf, never NaN
         const float *fv = h.bvh_kind == rt::BVH2 ? reinterpret_cast<const float *>(h.nodes2.data())
@@ -491,6 +493,17 @@ void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
             if (k % row < boxes && std::isnan(fv[k])) nan_free = false;
         s->desc.nan_free = nan_free ? 1 : 0;
     }
+}
+
+hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
+                      const rt::node4 *&nodes4) {
+    const rt::flat_scene &h = s->host;
+    nodes2 = h.nodes2.data();
+    nodes4 = h.nodes4.data();
+    if (h.bvh_kind != rt::BVH2 || h.nodes2.size() == s->n_nodes) return hipSuccess;
+    fetched.resize(s->n_nodes);
+    nodes2 = fetched.data();
+    return hipMemcpy(fetched.data(), s->nodes.p, sizeof(rt::node2) * s->n_nodes, hipMemcpyDeviceToHost);
 }
 
 } // namespace hiprt_detail
@@ -642,8 +655,8 @@ int hiprt_scene_layout(hiprt_scene sc, uint32_t *n_nodes, uint32_t *n_slots, int
                        int32_t *bvh_format, int32_t *tri_format) {
     if (!sc) return fail(HIPRT_ERR_ARG, "null scene");
     const rt::flat_scene &h = sc->host;
-    if (n_nodes) *n_nodes = (uint32_t)(h.bvh_kind == rt::BVH2 ? h.nodes2.size() : h.nodes4.size());
-    if (n_slots) *n_slots = (uint32_t)h.tris.size();
+    if (n_nodes) *n_nodes = sc->n_nodes;
+    if (n_slots) *n_slots = sc->n_slots;
     if (root_ref) *root_ref = h.root_ref;
     if (depth) *depth = h.depth;
     if (bvh_format) *bvh_format = h.bvh_kind;
@@ -658,8 +671,8 @@ int hiprt_scene_download(hiprt_scene sc, void *nodes, void *tri_records, uint32_
     // sizes of the layout (hiprt_scene_layout), not of the allocations, which
     // a device build makes for its worst case
     const rt::flat_scene &h = sc->host;
-    size_t node_bytes = h.bvh_kind == rt::BVH2 ? h.nodes2.size() * sizeof(rt::node2) : h.nodes4.size() * sizeof(rt::node4);
-    size_t rec_bytes = h.tris.size() * sizeof(rt::tri_rec), id_bytes = h.slot_ids.size() * 4;
+    size_t node_bytes = sc->n_nodes * (h.bvh_kind == rt::BVH2 ? sizeof(rt::node2) : sizeof(rt::node4));
+    size_t rec_bytes = sc->n_slots * sizeof(rt::tri_rec), id_bytes = 4ull * sc->n_slots;
     if (nodes && node_bytes) HIP_TRY(hipMemcpy(nodes, sc->nodes.p, node_bytes, hipMemcpyDeviceToHost));
     if (tri_records && rec_bytes) HIP_TRY(hipMemcpy(tri_records, sc->tris.p, rec_bytes, hipMemcpyDeviceToHost));
     if (slot_ids && id_bytes) HIP_TRY(hipMemcpy(slot_ids, sc->slot_ids.p, id_bytes, hipMemcpyDeviceToHost));
@@ -669,57 +682,55 @@ int hiprt_scene_download(hiprt_scene sc, void *nodes, void *tri_records, uint32_
 int hiprt_scene_refit(hiprt_scene sc, const float *d_positions, void *stream) {
     if (!sc || !d_positions) return fail(HIPRT_ERR_ARG, "null argument");
     if (!sc->tri_vidx.p) {
-        if (sc->host.tris.empty()) return ok();
+        if (sc->n_slots == 0) return ok();
         return fail(HIPRT_ERR_UNSUPPORTED, "refit needs a scene committed from a host scene");
     }
     HIP_TRY(hipSetDevice(sc->ctx->device));
     const rt::flat_scene &h = sc->host;
-    if (sc->refit_off.empty()) {
-        // inner nodes grouped by depth, deepest level first
-        std::vector<std::vector<int32_t>> levels;
-        if (h.root_ref >= 0) {
-            std::vector<int32_t> cur{h.root_ref};
-            while (!cur.empty()) {
-                levels.push_back(cur);
-                std::vector<int32_t> next;
-                for (int32_t id : cur) {
-                    int32_t refs[4] = {rt::kInvalidRef, rt::kInvalidRef, rt::kInvalidRef, rt::kInvalidRef};
-                    if (h.bvh_kind == rt::BVH2) {
-                        refs[0] = h.nodes2[id].ref_l;
-                        refs[1] = h.nodes2[id].ref_r;
-                    } else {
-                        for (int c = 0; c < 4; ++c) refs[c] = h.nodes4[id].ref[c];
-                    }
-                    for (int32_t r : refs)
-                        if (r >= 0 && r != rt::kInvalidRef) next.push_back(r);
-                }
-                cur.swap(next);
+    if (!sc->refit_boxes.p && sc->n_slots) {
+        // the slots below each child, children before their parents (their
+        // indices increase along every edge)
+        const uint32_t width = h.bvh_kind == rt::BVH2 ? 2u : 4u;
+        std::vector<rt::node2> fetched;
+        const rt::node2 *nodes2 = nullptr;
+        const rt::node4 *nodes4 = nullptr;
+        HIP_TRY(hiprt_detail::host_nodes(sc, fetched, nodes2, nodes4));
+        std::vector<uint2> ranges((size_t)width * sc->n_nodes, make_uint2(0, 0)), whole(sc->n_nodes);
+        for (size_t i = sc->n_nodes; i-- > 0;) {
+            uint32_t lo = 0xffffffffu, hi = 0, sum = 0;
+            for (uint32_t c = 0; c < width; ++c) {
+                const int32_t r = width == 2 ? (c ? nodes2[i].ref_r : nodes2[i].ref_l) : nodes4[i].ref[c];
+                if (r == rt::kInvalidRef) continue;
+                const uint2 q = rt::ref_is_leaf(r)
+                                    ? make_uint2(rt::leaf_slot(r), rt::leaf_slot(r) + rt::leaf_count(r))
+                                    : whole[r];
+                ranges[width * i + c] = q;
+                lo = std::min(lo, q.x);
+                hi = std::max(hi, q.y);
+                sum += q.y - q.x;
             }
+            // every builder partitions its triangle list in place
+            if (hi - lo != sum) return fail(HIPRT_ERR_UNSUPPORTED, "refit needs a tree whose subtrees are slot ranges");
+            whole[i] = make_uint2(lo, hi);
         }
-        std::vector<int32_t> list;
-        sc->refit_off.push_back(0);
-        for (auto it = levels.rbegin(); it != levels.rend(); ++it) {
-            list.insert(list.end(), it->begin(), it->end());
-            sc->refit_off.push_back((uint32_t)list.size());
-        }
-        HIP_TRY(sc->refit_list.upload(list.data(), list.size() * 4));
+        HIP_TRY(sc->refit_ranges.upload(ranges.data(), ranges.size() * sizeof(uint2)));
+        HIP_TRY(sc->refit_boxes.alloc(rt::dev::box_tree_entries(sc->n_slots) * sizeof(rt::dev::box6)));
     }
     rt::dev::refit_args a{};
     a.nodes = sc->nodes.p;
     a.bvh = h.bvh_kind;
+    a.n_nodes = sc->n_nodes;
     a.tris = sc->tris.as<rt::tri_rec>();
     a.slot_ids = sc->slot_ids.as<uint32_t>();
     a.tri = h.tri_kind;
-    a.n_slots = (uint32_t)h.tris.size();
+    a.n_slots = sc->n_slots;
     a.tri_geo = sc->tri_geo.as<float>();
     a.n_tris = sc->n_tris;
     a.pos = d_positions;
     a.vidx = sc->tri_vidx.as<uint32_t>();
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    HIP_TRY(rt::dev::launch_refit_records(a, s));
-    const int32_t *list = sc->refit_list.as<int32_t>();
-    for (size_t k = 0; k + 1 < sc->refit_off.size(); ++k)
-        HIP_TRY(rt::dev::launch_refit_level(a, list + sc->refit_off[k], sc->refit_off[k + 1] - sc->refit_off[k], s));
+    a.ranges = sc->refit_ranges.as<const uint2>();
+    a.boxes = sc->refit_boxes.as<rt::dev::box6>();
+    HIP_TRY(rt::dev::launch_refit(a, static_cast<hipStream_t>(stream)));
     sc->desc.nan_free = 1;   // select-based min/max from an empty box never store NaN
     return ok();
 }

@@ -31,18 +31,27 @@ inline int ok() { return HIPRT_OK; }
             return ::hiprt_detail::fail(HIPRT_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_));     \
     } while (0)
 
-// Owned device allocation.
+// Owned device allocation, or a view of a part of another one.
 struct dbuf {
     void *p = nullptr;
     size_t bytes = 0;
+    bool owned = true;
     dbuf() = default;
     dbuf(const dbuf &) = delete;
     dbuf &operator=(const dbuf &) = delete;
     ~dbuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p && owned) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
+        owned = true;
+    }
+    // The `n` bytes at `at` of an allocation that outlives this buffer.
+    void view(void *at, size_t n) {
+        release();
+        p = at;
+        bytes = n;
+        owned = false;
     }
     hipError_t alloc(size_t n) {
         release();
@@ -76,6 +85,10 @@ struct hiprt_stream_state {
     hiprt_detail::dbuf batch_table;   // descriptor table of the last batched trace on the stream
     hiprt_detail::dbuf spill;         // stack spill buffer of the persistent kernels (grown on demand)
     hiprt_detail::dbuf adjoint;       // sort scratch of the adjoint's vertex accumulation (grown on demand)
+    // device BVH builds: their scratch (bounded, kept between builds) and result words; one
+    // build at a time, which waits for its own work
+    std::mutex build_lock;
+    hiprt_detail::dbuf build_scratch, build_result;
 };
 
 struct hiprt_context_s {
@@ -89,7 +102,10 @@ struct hiprt_context_s {
 
 struct hiprt_scene_s {
     hiprt_context ctx = nullptr;
-    rt::flat_scene host;                         // host copy of the uploaded layout
+    rt::flat_scene host;                         // host copy of the uploaded layout (a scene built on the
+                                                 // device: its scalars only, see host_nodes)
+    uint32_t n_nodes = 0, n_slots = 0;
+    hiprt_detail::dbuf arena;                    // one allocation behind the buffers below (device builds)
     hiprt_detail::dbuf nodes, tris, slot_ids;    // traversal data
     hiprt_detail::dbuf tri_geo, mats;            // shading data (scenes committed from a host scene)
     hiprt_detail::dbuf tri_vidx;                 // vertex indices per triangle (adjoint scatter)
@@ -100,8 +116,7 @@ struct hiprt_scene_s {
     hiprt_detail::dbuf light_rec, light_f, light_cdf;   // light list of the direct-lighting steps
     uint32_t n_lights = 0;
     float light_integral = 0.0f;
-    hiprt_detail::dbuf refit_list;               // inner nodes by level, deepest first (refit)
-    std::vector<uint32_t> refit_off;             // level boundaries in refit_list
+    hiprt_detail::dbuf refit_ranges, refit_boxes;   // leaf slots below each child; box tree over the slots (refit)
     rt::scene_desc desc{};
 };
 
@@ -111,6 +126,11 @@ namespace hiprt_detail {
 // depth and node limits) and computes the most stack entries a traversal can
 // hold.  Returns "" when the tree is valid.
 std::string check_layout(rt::flat_scene &f, uint32_t &stack_need);
+
+// The scene's inner nodes on the host (references as committed; a scene built
+// on the device copies them into `fetched` from device memory).
+hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
+                      const rt::node4 *&nodes4);
 
 // Fills the scene descriptor from the device buffers and the host copy.
 void set_desc(hiprt_scene_s *s, uint32_t stack_need);

@@ -14,7 +14,8 @@ namespace dev {
 struct lbvh_in {
     const float *pos;        // 3 floats per vertex
     const uint32_t *vidx;    // 3 vertex indices per triangle
-    uint32_t n_vert, n_tris;
+    const uint32_t *mat;     // material id per triangle, or null (all 0)
+    uint32_t n_vert, n_tris, n_mats;
     int max_leaf;            // leaf size bound (1..32)
     int tri;                 // tri_format of the records
 };
@@ -23,9 +24,12 @@ struct lbvh_out {
     node2 *nodes;            // n_tris - 1 entries reserved (at most that many are written)
     tri_rec *tris;           // n_tris records, slot k = k-th triangle in Morton order
     uint32_t *slot_ids;      // n_tris
+    float *tri_geo;          // 12 floats per triangle: A.xyz + material bits, B.xyz, C.xyz (w words 0)
+    uint32_t *tri_vidx;      // copy of the 3 vertex indices per triangle
     int32_t *root_ref;       // device int32: root inner node 0, or the leaf reference of a one-leaf tree
-    uint32_t *counts;        // device uint32[4]: emitted inner nodes, depth (inner nodes on the longest path),
-                             // bad vertex indices, unused
+    uint32_t *counts;        // device uint32[5]: emitted inner nodes, depth (inner nodes on the longest path),
+                             // triangles with a bad vertex index, nodes that failed the layout check,
+                             // triangles with a bad material id
 };
 
 // Scratch the build needs, in bytes, for n_tris triangles.

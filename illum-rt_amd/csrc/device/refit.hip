@@ -2,16 +2,22 @@
 //
 // Records are rebuilt per leaf slot with the host flattener's own functions
 // (core/records.h), so a refit to the committed positions reproduces the
-// committed records bit for bit.  Boxes are recomputed bottom-up, one launch
-// per tree level (deepest first): a leaf child's box is the bounding box of
-// its triangles' vertices, an inner child's box the union of that child's own
-// child boxes.  Leaf boxes therefore bound whole triangles even where the
-// builder's early split clipping had bounded fragments (a fragment box lies
-// inside the triangle's box, so every hit stays reachable).
+// committed records bit for bit.  A leaf child's box is the bounding box of
+// its triangles' vertices, an inner child's box that of every triangle below
+// it.  Leaf boxes therefore bound whole triangles even where the builder's
+// early split clipping had bounded fragments (a fragment box lies inside the
+// triangle's box, so every hit stays reachable).
 //
-// Min/max are the select forms of glm::min/max (aabb::grow,
-// libgi/intersect.h:9-15) starting from an empty box (+inf, -inf); a NaN
-// coordinate never enters a box that way, so refit boxes are NaN-free.
+// The builders partition their triangle lists in place, so the slots below a
+// child are one range: its box is a range of the box tree (box_tree.h) that
+// the record kernel builds over the slots as it goes.  What bounds it is
+// latency: three launches, the gathers slot -> triangle -> vertices, and up to
+// 2 log2(slots) independent box loads per child.  One launch per tree level,
+// deepest first, took 22 dependent launches for the hall's tree (262,144
+// triangles): 155 us, this 40 us.
+//
+// Min/max are select forms that never let a NaN coordinate into a box, so
+// refit boxes are NaN-free.
 #include "refit_kernels.h"
 
 #include "../core/records.h"
@@ -21,79 +27,24 @@ namespace dev {
 
 namespace {
 
-struct dbox {
-    float lo[3], hi[3];
-};
-
-__device__ __forceinline__ dbox empty_box() {
-    return dbox{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
-}
-
-__device__ __forceinline__ void grow(dbox &b, float x, float y, float z) {
-    b.lo[0] = (x < b.lo[0]) ? x : b.lo[0];
-    b.lo[1] = (y < b.lo[1]) ? y : b.lo[1];
-    b.lo[2] = (z < b.lo[2]) ? z : b.lo[2];
-    b.hi[0] = (b.hi[0] < x) ? x : b.hi[0];
-    b.hi[1] = (b.hi[1] < y) ? y : b.hi[1];
-    b.hi[2] = (b.hi[2] < z) ? z : b.hi[2];
-}
-
-__device__ __forceinline__ void merge(dbox &b, const dbox &c) {
-    for (int k = 0; k < 3; ++k) {
-        b.lo[k] = (c.lo[k] < b.lo[k]) ? c.lo[k] : b.lo[k];
-        b.hi[k] = (b.hi[k] < c.hi[k]) ? c.hi[k] : b.hi[k];
-    }
-}
-
 __device__ __forceinline__ vec3f vertex(const float *pos, uint32_t v) {
     return vec3f{pos[3ull * v], pos[3ull * v + 1], pos[3ull * v + 2]};
 }
 
-__device__ __forceinline__ uint32_t slot_triangle(const refit_args &a, uint32_t slot) {
-    return a.slot_ids[slot];
-}
-
-__device__ dbox leaf_box(const refit_args &a, int32_t ref) {
-    dbox b = empty_box();
-    uint32_t slot = leaf_slot(ref), cnt = leaf_count(ref);
-    for (uint32_t k = 0; k < cnt; ++k) {
-        uint32_t t = slot_triangle(a, slot + k);
-        for (int c = 0; c < 3; ++c) {
-            vec3f p = vertex(a.pos, a.vidx[3ull * t + c]);
-            grow(b, p.x, p.y, p.z);
-        }
-    }
-    return b;
-}
-
-// Union of the child boxes stored in inner node `i`.
-__device__ dbox inner_box(const refit_args &a, int32_t i) {
-    dbox b = empty_box();
-    if (a.bvh == BVH2) {
-        const node2 &n = static_cast<const node2 *>(a.nodes)[i];
-        merge(b, dbox{{n.lxlo, n.lylo, n.lzlo}, {n.lxhi, n.lyhi, n.lzhi}});
-        merge(b, dbox{{n.rxlo, n.rylo, n.rzlo}, {n.rxhi, n.ryhi, n.rzhi}});
-    } else {
-        const node4 &n = static_cast<const node4 *>(a.nodes)[i];
-        for (int c = 0; c < 4; ++c)
-            if (n.ref[c] != kInvalidRef) merge(b, dbox{{n.lox[c], n.loy[c], n.loz[c]}, {n.hix[c], n.hiy[c], n.hiz[c]}});
-    }
-    return b;
-}
-
-__device__ __forceinline__ dbox child_box(const refit_args &a, int32_t ref) {
-    if (ref == kInvalidRef) return empty_box();
-    return ref_is_leaf(ref) ? leaf_box(a, ref) : inner_box(a, ref);
-}
-
-__global__ __launch_bounds__(256) void k_refit_records(refit_args a) {
-    uint32_t i = blockIdx.x * 256u + threadIdx.x;
+// One thread per slot (and per triangle, for the shading copy).
+__global__ __launch_bounds__(kBoxBlock) void k_refit_records(refit_args a) {
+    const uint32_t i = blockIdx.x * (uint32_t)kBoxBlock + threadIdx.x;
+    box6 box = empty_box6();
     if (i < a.n_slots) {
         uint32_t t = a.slot_ids[i];
         vec3f A = vertex(a.pos, a.vidx[3ull * t]);
         vec3f B = vertex(a.pos, a.vidx[3ull * t + 1]);
         vec3f C = vertex(a.pos, a.vidx[3ull * t + 2]);
         a.tris[i] = a.tri == TRI_WOOP ? make_woop_rec(A, B, C) : make_exact_rec(A, B, C, t);
+        box_grow(box, A.x, A.y, A.z);
+        box_grow(box, B.x, B.y, B.z);
+        box_grow(box, C.x, C.y, C.z);
+        a.boxes[i] = box;
     }
     if (a.tri_geo && i < a.n_tris) {
         float *g = a.tri_geo + 12ull * i;
@@ -104,53 +55,51 @@ __global__ __launch_bounds__(256) void k_refit_records(refit_args a) {
             g[4 * c + 2] = p.z;
         }
     }
+    if (blockIdx.x * (uint32_t)kBoxBlock < a.n_slots) box_levels(box, a.boxes, a.n_slots);   // uniform per block
 }
 
-__global__ __launch_bounds__(256) void k_refit_level(refit_args a, const int32_t *list, uint32_t n) {
-    uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    int32_t id = list[i];
+// One thread per child.
+__global__ __launch_bounds__(256) void k_refit_nodes(refit_args a) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t width = a.bvh == BVH2 ? 2u : 4u;
+    if (i >= a.n_nodes * width) return;
+    const uint2 r = a.ranges[i];
+    const box6 b = box_of_range(a.boxes, a.n_slots, r.x, r.y);
     if (a.bvh == BVH2) {
-        node2 &nd = static_cast<node2 *>(a.nodes)[id];
-        dbox l = child_box(a, nd.ref_l), r = child_box(a, nd.ref_r);
-        nd.lxlo = l.lo[0];
-        nd.lxhi = l.hi[0];
-        nd.lylo = l.lo[1];
-        nd.lyhi = l.hi[1];
-        nd.lzlo = l.lo[2];
-        nd.lzhi = l.hi[2];
-        nd.rxlo = r.lo[0];
-        nd.rxhi = r.hi[0];
-        nd.rylo = r.lo[1];
-        nd.ryhi = r.hi[1];
-        nd.rzlo = r.lo[2];
-        nd.rzhi = r.hi[2];
-    } else {
-        node4 &nd = static_cast<node4 *>(a.nodes)[id];
-        for (int c = 0; c < 4; ++c) {
-            dbox b = child_box(a, nd.ref[c]);
-            nd.lox[c] = b.lo[0];
-            nd.hix[c] = b.hi[0];
-            nd.loy[c] = b.lo[1];
-            nd.hiy[c] = b.hi[1];
-            nd.loz[c] = b.lo[2];
-            nd.hiz[c] = b.hi[2];
+        node2 &nd = static_cast<node2 *>(a.nodes)[i >> 1];
+        float4 xy = make_float4(b.lo[0], b.hi[0], b.lo[1], b.hi[1]);
+        float2 z = make_float2(b.lo[2], b.hi[2]);
+        if (i & 1u) {
+            *reinterpret_cast<float4 *>(&nd.rxlo) = xy;
+            *reinterpret_cast<float2 *>(&nd.rzlo) = z;
+        } else {
+            *reinterpret_cast<float4 *>(&nd.lxlo) = xy;
+            *reinterpret_cast<float2 *>(&nd.lzlo) = z;
         }
+    } else {
+        node4 &nd = static_cast<node4 *>(a.nodes)[i >> 2];
+        const uint32_t c = i & 3u;
+        nd.lox[c] = b.lo[0];
+        nd.hix[c] = b.hi[0];
+        nd.loy[c] = b.lo[1];
+        nd.hiy[c] = b.hi[1];
+        nd.loz[c] = b.lo[2];
+        nd.hiz[c] = b.hi[2];
     }
 }
 
 } // namespace
 
-hipError_t launch_refit_records(const refit_args &a, hipStream_t stream) {
-    uint32_t n = a.n_slots > a.n_tris ? a.n_slots : a.n_tris;
+hipError_t launch_refit(const refit_args &a, hipStream_t stream) {
+    const uint32_t n = a.n_slots > a.n_tris ? a.n_slots : a.n_tris;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_refit_records, dim3((n + 255) / 256), dim3(256), 0, stream, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_refit_level(const refit_args &a, const int32_t *list, uint32_t n, hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_refit_level, dim3((n + 255) / 256), dim3(256), 0, stream, a, list, n);
+    hipLaunchKernelGGL(k_refit_records, dim3((n + kBoxBlock - 1) / kBoxBlock), dim3(kBoxBlock), 0, stream, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || a.n_nodes == 0) return e;
+    e = launch_box_tree_top(a.boxes, a.n_slots, stream);
+    if (e != hipSuccess) return e;
+    const uint32_t children = a.n_nodes * (a.bvh == BVH2 ? 2u : 4u);
+    hipLaunchKernelGGL(k_refit_nodes, dim3((children + 255) / 256), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

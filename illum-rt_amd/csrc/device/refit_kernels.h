@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../core/layout.h"
+#include "box_tree.h"
 
 #include <cstdint>
 
@@ -14,6 +15,7 @@ namespace dev {
 struct refit_args {
     void *nodes;               // node2[] or node4[]
     int bvh;                   // bvh_format
+    uint32_t n_nodes;
     tri_rec *tris;             // one record per leaf slot
     const uint32_t *slot_ids;  // slot -> triangle id
     int tri;                   // tri_format
@@ -22,15 +24,13 @@ struct refit_args {
     uint32_t n_tris;
     const float *pos;          // 3 floats per vertex
     const uint32_t *vidx;      // 3 vertex indices per triangle
+    const uint2 *ranges;       // leaf slots [x, y) below each child, 2 or 4 per node (empty: absent child)
+    box6 *boxes;               // box_tree_entries(n_slots)
 };
 
-// Rewrites every triangle record (and the shading copy of the vertices) from
-// `pos`.
-hipError_t launch_refit_records(const refit_args &a, hipStream_t stream);
-
-// Recomputes the child boxes of the `n` inner nodes listed at `list`; each
-// listed node's inner children must already be final.
-hipError_t launch_refit_level(const refit_args &a, const int32_t *list, uint32_t n, hipStream_t stream);
+// Records, shading vertices and every node box from the new positions: three
+// launches up to a million slots.
+hipError_t launch_refit(const refit_args &a, hipStream_t stream);
 
 } // namespace dev
 } // namespace rt

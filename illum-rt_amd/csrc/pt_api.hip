@@ -32,7 +32,8 @@ namespace {
 
 // Sort grid over the scene box: the union of the root's child boxes (a
 // one-leaf or empty tree sorts by the direction's cell or octant only).
-rt::dev::sort_grid grid_of(const rt::flat_scene &h) {
+hipError_t grid_of(const hiprt_scene_s *sc, rt::dev::sort_grid *out) {
+    const rt::flat_scene &h = sc->host;
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     auto grow = [&](float xl, float xh, float yl, float yh, float zl, float zh) {
         lo[0] = std::min(lo[0], xl);
@@ -42,8 +43,14 @@ rt::dev::sort_grid grid_of(const rt::flat_scene &h) {
         hi[1] = std::max(hi[1], yh);
         hi[2] = std::max(hi[2], zh);
     };
-    if (h.root_ref >= 0 && h.bvh_kind == rt::BVH2 && (size_t)h.root_ref < h.nodes2.size()) {
-        const rt::node2 &r = h.nodes2[h.root_ref];
+    if (h.root_ref >= 0 && h.bvh_kind == rt::BVH2 && (uint32_t)h.root_ref < sc->n_nodes) {
+        rt::node2 r;
+        if (h.nodes2.empty()) {   // built on the device
+            hipError_t e = hipMemcpy(&r, sc->nodes.as<const rt::node2>() + h.root_ref, sizeof r, hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return e;
+        } else {
+            r = h.nodes2[h.root_ref];
+        }
         grow(r.lxlo, r.lxhi, r.lylo, r.lyhi, r.lzlo, r.lzhi);
         grow(r.rxlo, r.rxhi, r.rylo, r.ryhi, r.rzlo, r.rzhi);
     } else if (h.root_ref >= 0 && h.bvh_kind == rt::BVH4 && (size_t)h.root_ref < h.nodes4.size()) {
@@ -59,7 +66,8 @@ rt::dev::sort_grid grid_of(const rt::flat_scene &h) {
         g.scale[a] = ok_axis ? (float)(1u << rt::dev::kSortCellBits) / ext : 0.0f;
         if (!std::isfinite(g.scale[a])) g.scale[a] = 0.0f;
     }
-    return g;
+    *out = g;
+    return hipSuccess;
 }
 
 // Shading data of a committed scene for the device steps.
@@ -714,7 +722,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
         HIP_TRY(p->perm.alloc(4ull * n));
         HIP_TRY(p->sort_counts.alloc(4ull * 256 * rt::dev::radix_tiles(n)));
         HIP_TRY(p->sort_totals.alloc(4ull * 256));
-        p->grid = grid_of(sc->host);
+        HIP_TRY(grid_of(sc, &p->grid));
     }
     if (p->batched) {
         // Resolve the persistent grid size outside the capture, then record

@@ -197,8 +197,8 @@ int hiprt_scene_commit(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, int32
  * (rt/cuda/base.cpp:88-117).  This tree is not the reference's SAH tree:
  * hits agree with brute force up to equal-t ties and grazing hits.
  * *device_ms (optional) receives the build kernels' time on `stream`; the
- * call returns after the scene is ready (it copies the flattened tree back
- * to the host once to check it). */
+ * call returns after the scene is ready; the tree is checked and stays on the
+ * device. */
 int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_vert, const uint32_t *d_indices,
                       uint32_t n_tris, const uint32_t *d_materials, const float *materials, uint32_t n_materials,
                       int32_t max_leaf, int32_t tri_format, hiprt_scene *out, float *device_ms, void *stream);
@@ -218,8 +218,8 @@ int hiprt_scene_layout(hiprt_scene sc, uint32_t *n_nodes, uint32_t *n_slots, int
 int hiprt_scene_download(hiprt_scene sc, void *nodes, void *tri_records, uint32_t *slot_ids);
 /* Refit to new vertex positions (d_positions: 3 floats per vertex, as many
  * vertices as the committed host scene): same triangles and tree topology,
- * triangle records rebuilt, node boxes recomputed bottom-up on the device,
- * one launch per tree level.  Leaf boxes bound whole triangles.  The device
+ * triangle records rebuilt, node boxes recomputed on the device from a tree
+ * of boxes over the leaf slots (three launches).  Leaf boxes bound whole triangles.  The device
  * counterpart of rebuilding on every commit (rt/cuda/base.cpp:88-117) when
  * only vertices move -- scene-view transforms (rt/cuda/preprocessing.cpp:41-72)
  * or gradient steps on vertices.  Needs a scene from hiprt_scene_commit;
