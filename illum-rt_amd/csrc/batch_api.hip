@@ -200,6 +200,7 @@ int hiprt_autotune(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, const hip
                                                                                      : std::vector<int>{40};
             hiprt_tracer_opts base{40, 0, nullptr, stack, 1, 0, 0};
             rt::dev::persistent_cfg pc = cfg_for(tracer, &base);
+            pc.need = layouts[f]->stack_need;
             int full = 0;
             HIP_TRY(rt::dev::persistent_grid(layouts[f]->desc, any != 0, pc, &full));
             for (int thr : thresholds)

@@ -51,6 +51,8 @@ rt::scene_desc desc_for(const hiprt_scene_s *sc, bool alpha) {
 hipError_t attach_spill(hiprt_stream_state *st, hipStream_t s, const rt::scene_desc &d, bool any, bool multi,
                         int need, rt::dev::persistent_cfg &cfg, int spill_limit) {
     cfg.spill = nullptr;
+    cfg.need = spill_limit > 0 ? 0 : need;
+    if (rt::dev::dynamic_fits(d.bvh, any, multi, cfg)) return hipSuccess;   // its stack is in LDS
     cfg.spill_cap = rt::dev::persistent_spill_entries(d.bvh, cfg.stack, need);
     if (spill_limit > 0 && cfg.spill_cap > (uint32_t)spill_limit) cfg.spill_cap = (uint32_t)spill_limit;
     cfg.spill_bytes = 0;

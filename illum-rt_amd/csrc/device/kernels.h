@@ -87,6 +87,7 @@ struct persistent_cfg {
     int32_t *spill = nullptr;
     uint32_t spill_cap = 0;
     size_t spill_bytes = 0;
+    int need = 0;         // the trees' stack need; 0: not known, or the caller bounds the spill column
 };
 
 // `counter` points to kCounterBytes of device memory (cleared by the launch);
@@ -98,6 +99,20 @@ hipError_t launch_trace_persistent(const scene_desc &sc, const ray_soa &rays, co
                                    uint8_t *occluded, uint32_t n, const uint32_t *count_ptr, uint32_t *counter,
                                    bool any, const persistent_cfg &cfg, hipStream_t stream,
                                    ray_gather gather = ray_gather{});
+
+// The postponing tracers of binary trees, with the tree's whole stack in LDS
+// (trace_dynamic.hip): any-hit of one scene, and descriptor tables.  Does a
+// launch of this kind take it?  Trees of more entries, launches that count
+// fetches and those whose caller bounds the spill column keep the kernels of
+// trace_persistent.hip, which call these.
+constexpr int kDynamicStackNeed = 32;
+bool dynamic_fits(int bvh, bool any, bool multi, const persistent_cfg &cfg);
+hipError_t dynamic_grid(int tri, bool any, bool multi, const persistent_cfg &cfg, int *blocks);
+hipError_t launch_trace_dynamic(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,
+                                uint32_t n, const uint32_t *count_ptr, uint32_t *counter, const persistent_cfg &cfg,
+                                hipStream_t stream, ray_gather gather);
+hipError_t launch_trace_dynamic_batch(const batch_desc *d_table, uint32_t n_desc, uint32_t total, int tri, bool any,
+                                      uint32_t *counter, const persistent_cfg &cfg, hipStream_t stream);
 
 // One persistent launch over a descriptor table (device memory, sorted by
 // `first`, first entry at 0, `total` rays in all).  All scenes must share the

@@ -14,6 +14,7 @@
 
 #include "../core/layout.h"
 #include "../core/raygen.h"
+#include "kernels.h"
 
 #include <cfloat>
 #include <cstdint>
@@ -128,6 +129,44 @@ __device__ __forceinline__ bool ray_is_finite(const dray &r) {
            !isnan(r.tmax);
 }
 
+// IEEE minimum and maximum of values that are not signalling NaNs, without
+// the canonicalizing instructions fminf and fmaxf bring along.
+__device__ __forceinline__ float min_of(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max_of(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min3_of(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float max3_of(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// box_fast on those.
+template <bool ANY>
+__device__ __forceinline__ bool box_min3(float xlo, float xhi, float ylo, float yhi, float zlo, float zhi,
+                                         const dray &r, float best, float &dist) {
+    float ax = (xlo - r.ox) * r.ix, bx = (xhi - r.ox) * r.ix;
+    float ay = (ylo - r.oy) * r.iy, by = (yhi - r.oy) * r.iy;
+    float az = (zlo - r.oz) * r.iz, bz = (zhi - r.oz) * r.iz;
+    float t1 = max3_of(min_of(ax, bx), min_of(ay, by), min_of(az, bz));
+    float t2 = min3_of(max_of(ax, bx), max_of(ay, by), max_of(az, bz));
+    dist = t1;
+    bool hit = (t1 <= t2) && (t2 >= r.tmin) && (t1 <= r.tmax);
+    if (!ANY) hit = hit && (t1 < best);
+    return hit;
+}
+
 template <bool ANY>
 __device__ __forceinline__ bool box_test(bool exact, float xlo, float xhi, float ylo, float yhi, float zlo,
                                          float zhi, const dray &r, float best, float &dist) {
@@ -199,6 +238,8 @@ __device__ __forceinline__ bool tri_woop(const float4 &m0, const float4 &m1, con
     return true;
 }
 
+__device__ __forceinline__ uint64_t wave_mask(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
 __device__ __forceinline__ uint32_t as_u32(float f) { return __float_as_uint(f); }
 
 // Texel of texture2d::sample (libgi/scene.h:28-36): wrap by subtracting the
@@ -254,6 +295,18 @@ __device__ __forceinline__ uint32_t slot_tri_id(const scene_desc &sc, uint32_t s
 // still descend: the lanes that hold a leaf do not wait for the last few.
 // Each lane's own order is unchanged.  (Measured beside k_trace_plain.)
 constexpr int kNodeLanes = 8;
+
+// Index of the descriptor whose ray range holds global ray `idx`
+// (descriptors sorted by `first`, the first starting at 0).
+__device__ __forceinline__ uint32_t find_desc(const batch_desc *table, uint32_t n_desc, uint32_t idx) {
+    uint32_t lo = 0, hi = n_desc;
+    while (hi - lo > 1) {
+        uint32_t mid = (lo + hi) >> 1;
+        if (table[mid].first <= idx) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
 
 // Result of one ray.
 struct dhit {

@@ -71,63 +71,13 @@ struct group_args {
     uint32_t cap, soft;   // entries per ray; list length up to which steps take K entries
 };
 
-__device__ __forceinline__ uint32_t find_desc(const batch_desc *table, uint32_t n_desc, uint32_t idx) {
-    uint32_t lo = 0, hi = n_desc;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (table[mid].first <= idx) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
-__device__ __forceinline__ uint64_t wave_mask(bool p) { return __builtin_amdgcn_ballot_w64(p); }
-
 // This group's bits of a wave mask.
 template <int K> __device__ __forceinline__ uint32_t group_bits(uint64_t mask, uint32_t shift) {
     return (uint32_t)(mask >> shift) & ((1u << K) - 1u);
 }
 
-// IEEE minimum and maximum of values that are not signalling NaNs, without
-// the canonicalizing instructions fminf and fmaxf bring along.
-__device__ __forceinline__ float min_of(float a, float b) {
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float max_of(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float min3_of(float a, float b, float c) {
-    float r;
-    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float max3_of(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 template <int CTRL> __device__ __forceinline__ float dpp(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-
-// box_fast (trace_core.h) on those.
-template <bool ANY>
-__device__ __forceinline__ bool box_min3(float xlo, float xhi, float ylo, float yhi, float zlo, float zhi,
-                                         const dray &r, float best, float &dist) {
-    float ax = (xlo - r.ox) * r.ix, bx = (xhi - r.ox) * r.ix;
-    float ay = (ylo - r.oy) * r.iy, by = (yhi - r.oy) * r.iy;
-    float az = (zlo - r.oz) * r.iz, bz = (zhi - r.oz) * r.iz;
-    float t1 = max3_of(min_of(ax, bx), min_of(ay, by), min_of(az, bz));
-    float t2 = min3_of(max_of(ax, bx), max_of(ay, by), max_of(az, bz));
-    dist = t1;
-    bool hit = (t1 <= t2) && (t2 >= r.tmin) && (t1 <= r.tmax);
-    if (!ANY) hit = hit && (t1 < best);
-    return hit;
 }
 
 } // namespace

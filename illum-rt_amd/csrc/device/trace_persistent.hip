@@ -185,18 +185,6 @@ __device__ __forceinline__ void cswap(float &ka, int32_t &ra, float &kb, int32_t
     }
 }
 
-// Index of the descriptor whose ray range holds global ray `idx`
-// (descriptors sorted by `first`, the first starting at 0).
-__device__ __forceinline__ uint32_t find_desc(const batch_desc *table, uint32_t n_desc, uint32_t idx) {
-    uint32_t lo = 0, hi = n_desc;
-    while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (table[mid].first <= idx) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 } // namespace
 
 // Waves per SIMD the register allocation must leave room for: 8 for
@@ -625,6 +613,7 @@ size_t persistent_spill_bytes(int blocks, uint32_t entries) {
 }
 
 hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg &cfg, int *blocks, bool multi) {
+    if (dynamic_fits(sc.bvh, any, multi, cfg)) return dynamic_grid(sc.tri, any, multi, cfg, blocks);
     launch_args a{};
     if (multi) return dispatch<true>(sc.tri, any, sc.bvh, a, cfg, nullptr, true, blocks);
     return dispatch<false>(sc.tri, any, sc.bvh, a, cfg, nullptr, true, blocks);
@@ -635,6 +624,8 @@ hipError_t launch_trace_persistent(const scene_desc &sc, const ray_soa &rays, co
                                    bool any, const persistent_cfg &cfg, hipStream_t stream, ray_gather gather) {
     hipError_t e = launch_fill_u32(counter, 0u, kMaxChunks * kCounterStride, stream);
     if (e != hipSuccess) return e;
+    if (dynamic_fits(sc.bvh, any, false, cfg))
+        return launch_trace_dynamic(sc, rays, hits, occluded, n, count_ptr, counter, cfg, stream, gather);
     launch_args a{sc, rays, gather, hits, occluded, n, count_ptr, counter, nullptr, 0};
     return dispatch<false>(sc.tri, any, sc.bvh, a, cfg, stream, false, nullptr);
 }
@@ -643,6 +634,8 @@ hipError_t launch_trace_batch(const batch_desc *d_table, uint32_t n_desc, uint32
                               uint32_t *counter, const persistent_cfg &cfg, hipStream_t stream) {
     hipError_t e = launch_fill_u32(counter, 0u, kMaxChunks * kCounterStride, stream);
     if (e != hipSuccess) return e;
+    if (dynamic_fits(bvh, any, true, cfg))
+        return launch_trace_dynamic_batch(d_table, n_desc, total, tri, any, counter, cfg, stream);
     launch_args a{};
     a.n = total;
     a.counter = counter;
