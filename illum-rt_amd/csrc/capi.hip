@@ -472,6 +472,20 @@ std::string check_layout(rt::flat_scene &f, uint32_t &stack_need) {
     return "";
 }
 
+// Does every child's box hold the boxes stored in that child?  (NaN: no.)
+static bool boxes_nested(const std::vector<rt::node2> &nodes) {
+    auto inside = [](const rt::node2 &c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi) {
+        return c.lxlo >= xlo && c.lxhi <= xhi && c.lxlo <= c.lxhi && c.rxlo >= xlo && c.rxhi <= xhi && c.rxlo <= c.rxhi &&
+               c.lylo >= ylo && c.lyhi <= yhi && c.lylo <= c.lyhi && c.rylo >= ylo && c.ryhi <= yhi && c.rylo <= c.ryhi &&
+               c.lzlo >= zlo && c.lzhi <= zhi && c.lzlo <= c.lzhi && c.rzlo >= zlo && c.rzhi <= zhi && c.rzlo <= c.rzhi;
+    };
+    for (const rt::node2 &n : nodes) {
+        if (!rt::ref_is_leaf(n.ref_l) && !inside(nodes[n.ref_l], n.lxlo, n.lxhi, n.lylo, n.lyhi, n.lzlo, n.lzhi)) return false;
+        if (!rt::ref_is_leaf(n.ref_r) && !inside(nodes[n.ref_r], n.rxlo, n.rxhi, n.rylo, n.ryhi, n.rzlo, n.rzhi)) return false;
+    }
+    return true;
+}
+
 void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
     const rt::flat_scene &h = s->host;
     s->desc.nodes = s->nodes.p;
@@ -495,6 +509,7 @@ void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
             if (k % row < boxes && std::isnan(fv[k])) nan_free = false;
         s->desc.nan_free = nan_free ? 1 : 0;
     }
+    s->desc.nested = h.bvh_kind == rt::BVH2 && boxes_nested(h.nodes2) ? 1 : 0;
 }
 
 hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
@@ -734,6 +749,7 @@ int hiprt_scene_refit(hiprt_scene sc, const float *d_positions, void *stream) {
     a.boxes = sc->refit_boxes.as<rt::dev::box6>();
     HIP_TRY(rt::dev::launch_refit(a, static_cast<hipStream_t>(stream)));
     sc->desc.nan_free = 1;   // select-based min/max from an empty box never store NaN
+    sc->desc.nested = h.bvh_kind == rt::BVH2 ? 1 : 0;   // unions; a subtree of empty boxes holds no triangle to hit
     return ok();
 }
 

@@ -98,6 +98,8 @@ struct scene_desc {
     const void *alpha_tex;    // uint4
     const uint8_t *alpha_mask;
     int32_t alpha;
+    int32_t nested;           // binary tree whose child boxes lie inside their parents' (kernels may postpone leaves
+                              // and still return the reference's hits, see device/trace_plain.hip)
 };
 
 } // namespace rt

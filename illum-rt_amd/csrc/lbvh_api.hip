@@ -117,6 +117,7 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     sc->n_nodes = counts[0];
     sc->n_slots = n;
     sc->desc.nan_free = 1;
+    sc->desc.nested = 1;   // unions; a subtree of empty boxes holds no triangle to hit
     sc->n_tris = n;
     sc->n_vert = n_vert;
     *out = sc.release();
