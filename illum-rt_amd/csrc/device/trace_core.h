@@ -101,28 +101,8 @@ __device__ __forceinline__ bool box_exact(float xlo, float xhi, float ylo, float
     return hit;
 }
 
-// intersect4 when no slab value can be NaN: the operands are the same
-// separately rounded (box - o) * (1/d) products, and for NaN-free inputs the
-// select chains of intersect4 equal IEEE min/max (min3/max3 on gfx950),
-// differing at most in the sign of a zero, which no comparison sees.  NaN
-// slab values need a non-finite ray component or box bound; kernels take
-// this path only for wavefronts whose rays and scene are all finite.
-template <bool ANY>
-__device__ __forceinline__ bool box_fast(float xlo, float xhi, float ylo, float yhi, float zlo, float zhi,
-                                         const dray &r, float best, float &dist) {
-    float ax = (xlo - r.ox) * r.ix, bx = (xhi - r.ox) * r.ix;
-    float ay = (ylo - r.oy) * r.iy, by = (yhi - r.oy) * r.iy;
-    float az = (zlo - r.oz) * r.iz, bz = (zhi - r.oz) * r.iz;
-    float t1 = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz));
-    float t2 = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz));
-    dist = t1;
-    bool hit = (t1 <= t2) && (t2 >= r.tmin) && (t1 <= r.tmax);
-    if (!ANY) hit = hit && (t1 < best);
-    return hit;
-}
-
 // True when every component of the ray and of its inverse direction is
-// finite, i.e. box_fast decides exactly like box_exact for this ray.
+// finite, i.e. box_min3 decides exactly like box_exact for this ray.
 __device__ __forceinline__ bool ray_is_finite(const dray &r) {
     return isfinite(r.ox) && isfinite(r.oy) && isfinite(r.oz) && isfinite(r.dx) && isfinite(r.dy) &&
            isfinite(r.dz) && isfinite(r.ix) && isfinite(r.iy) && isfinite(r.iz) && !isnan(r.tmin) &&
@@ -152,7 +132,12 @@ __device__ __forceinline__ float max3_of(float a, float b, float c) {
     return r;
 }
 
-// box_fast on those.
+// intersect4 when no slab value can be NaN: the operands are the same
+// separately rounded (box - o) * (1/d) products, and for NaN-free inputs the
+// select chains of intersect4 equal IEEE min/max (min3/max3 on gfx950),
+// differing at most in the sign of a zero, which no comparison sees.  NaN
+// slab values need a non-finite ray component or box bound; kernels take
+// this path only for wavefronts whose rays and scene are all finite.
 template <bool ANY>
 __device__ __forceinline__ bool box_min3(float xlo, float xhi, float ylo, float yhi, float zlo, float zhi,
                                          const dray &r, float best, float &dist) {
@@ -171,7 +156,7 @@ template <bool ANY>
 __device__ __forceinline__ bool box_test(bool exact, float xlo, float xhi, float ylo, float yhi, float zlo,
                                          float zhi, const dray &r, float best, float &dist) {
     if (exact) return box_exact<ANY>(xlo, xhi, ylo, yhi, zlo, zhi, r, best, dist);
-    return box_fast<ANY>(xlo, xhi, ylo, yhi, zlo, zhi, r, best, dist);
+    return box_min3<ANY>(xlo, xhi, ylo, yhi, zlo, zhi, r, best, dist);
 }
 
 // Shirley/Cramer test on an exact record (A, A-B, A-C).  Accepts iff
