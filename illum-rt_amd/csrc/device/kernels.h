@@ -141,6 +141,15 @@ hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg 
 // A path tracer's later levels hold ever fewer of its slots: kGroupSlots8.
 // Whole frames: 1280 x 720 (921k) 4.19 ms, dynamic 4.83; 320 x 240 x 16
 // samples (1.23M) 5.41 against 5.82.
+// Up to kAppendSlots of them the group trace takes the later levels' records in
+// the order they were appended: a group's lanes share one ray, so sorting
+// buys less than its six launches a level.  Whole frames of 5 levels, us,
+// sorted / not: hall 480 x 270 1045 / 906, 640 x 480 1770 / 1665, 1120 x 630
+// (706k) 3340 / 3285, 1280 x 720 (922k) 4170 / 4180, 480 x 270 x 8 samples
+// (1.04M) 4555 / 4610; the 8,192-triangle scene 650 / 506, 1070 / 931, 2010 /
+// 1878, 2525 / 2395, 2890 / 2660; 2 slots per pixel for 8 samples of 480 x 270
+// 7030 / 6060 and 4995 / 3460.
+constexpr uint32_t kAppendSlots = 7u << 17;
 constexpr int kGroupStackNeed = 64;
 constexpr uint32_t kGroupRays16 = 1u << 16;
 constexpr uint32_t kGroupRays8 = 1u << 20;

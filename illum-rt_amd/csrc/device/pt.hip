@@ -329,7 +329,8 @@ __device__ __forceinline__ uint32_t octant_key(const sort_grid &g, vec3f o, vec3
 // they are null); later, direction and (path id bits, throughput) from record
 // src of in_rec.  The last level reads no direction: it only adds emission.
 // The hit is slot i.  Live
-// next-level rays are appended as records to out_rec with their keys: the
+// next-level rays are appended as records to out_rec with their keys (no
+// keys where the queue is not sorted): the
 // throughput travels with the ray, so no step reads or writes per-pixel
 // throughput at a random address.
 __global__ __launch_bounds__(kShadeBlock) void k_shade_stage(pt_scene ps, pt_params pp, int level,
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_stage(pt_scene ps, pt_par
         // the queue (their rays leave one point in many directions), the
         // octant over a 16^3 grid for one sample per pixel: each traced its
         // queue fastest in that setting
-        keys[slot] = pp.px_samples > 1 ? ray_key(grid, so.org, so.dir) : octant_key(grid, so.org, so.dir);
+        if (keys) keys[slot] = pp.px_samples > 1 ? ray_key(grid, so.org, so.dir) : octant_key(grid, so.org, so.dir);
     }
 }
 

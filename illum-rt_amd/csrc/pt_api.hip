@@ -124,6 +124,7 @@ struct hiprt_pt_s {
     // sorted bounce queues: ray records (ray, path id, throughput) per level
     // parity, keys, the permutation, and the radix sort's scratch
     bool sorted = false;
+    bool append_order = false;   // the group trace takes the records in the order they were appended: no sort
     dbuf rec[2], keys, keys_tmp, vals_tmp, perm, sort_counts, sort_totals;
     rt::dev::sort_grid grid{};
     rt::hit_soa h{};
@@ -178,19 +179,20 @@ struct hiprt_pt_s {
         using namespace rt::dev;
         uint32_t *q = qcount.as<uint32_t>();
         const regen_params rp = regen();
+        const bool reorder = sorted && !append_order;
         for (int it = 0; it < kRegenChunk; ++it) {
             const int a = it & 1, b = a ^ 1;
             ray_gather g;
             g.aos = rec[a].as<const float4>();
-            g.perm = sorted ? perm.as<const uint32_t>() : nullptr;
+            g.perm = reorder ? perm.as<const uint32_t>() : nullptr;
             g.stride = kRayRecord;
             g.fixed_t = 1;
             hipError_t e = trace(rt::ray_soa{}, q + a, pcfg, s, g);
             if (e == hipSuccess) e = launch_fill_u32(q + b, 0u, 1u, s);
             if (e == hipSuccess)
                 e = launch_shade_regen(ps(), pp, rp, rec[a].as<const float4>(), g.perm, h, rec[b].as<float4>(),
-                                       sorted ? keys.as<uint32_t>() : nullptr, q + a, q + b, grid, n, s);
-            if (e == hipSuccess && sorted) e = launch_radix_sort(sort_buffers(), n, q + b, regen_key_bits(lanes), s);
+                                       reorder ? keys.as<uint32_t>() : nullptr, q + a, q + b, grid, n, s);
+            if (e == hipSuccess && reorder) e = launch_radix_sort(sort_buffers(), n, q + b, regen_key_bits(lanes), s);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
@@ -205,8 +207,9 @@ struct hiprt_pt_s {
         HIP_TRY(launch_fill_u32(counts.as<uint32_t>(), 0u, (uint32_t)levels + 1, s));
         HIP_TRY(launch_fill_u32(q, n, 1u, s));
         HIP_TRY(launch_fill_u32(q + 1, 0u, 1u, s));
-        HIP_TRY(launch_regen_init(regen(), rec[0].as<float4>(), sorted ? keys.as<uint32_t>() : nullptr, s));
-        if (sorted) HIP_TRY(launch_radix_sort(sort_buffers(), n, q, regen_key_bits(lanes), s));
+        const bool reorder = sorted && !append_order;
+        HIP_TRY(launch_regen_init(regen(), rec[0].as<float4>(), reorder ? keys.as<uint32_t>() : nullptr, s));
+        if (reorder) HIP_TRY(launch_radix_sort(sort_buffers(), n, q, regen_key_bits(lanes), s));
         // every slot ends within ceil(samples / lanes) paths of at most
         // max_depth + 1 iterations each
         const uint64_t bound = (uint64_t)((samples + lanes - 1) / lanes) * (uint64_t)levels;
@@ -244,6 +247,7 @@ struct hiprt_pt_s {
         using namespace rt::dev;
         uint32_t *cnt = counts.as<uint32_t>();
         int levels = pp.max_depth + 1;
+        const bool reorder = sorted && (stats || !append_order);   // counting traces are one ray per lane
         hipError_t e = launch_fill_u32(cnt, 0u, (uint32_t)levels + 1, s);
         if (e != hipSuccess) return e;
         e = launch_fill_u32(cnt, n, 1u, s);
@@ -297,7 +301,7 @@ struct hiprt_pt_s {
                     // the previous shade step's records through the sorted
                     // permutation
                     const float4 *in_rec = L > 0 ? rec[(L - 1) & 1].as<const float4>() : nullptr;
-                    const uint32_t *pm = L > 0 ? perm.as<const uint32_t>() : nullptr;
+                    const uint32_t *pm = L > 0 && reorder ? perm.as<const uint32_t>() : nullptr;
                     ray_gather g;
                     g.aos = in_rec;
                     g.perm = pm;
@@ -310,8 +314,8 @@ struct hiprt_pt_s {
                     }
                     e = launch_shade_stage(ps(), pp, L, fs, rays[0].out, nullptr, nullptr, in_rec, pm, h,
                                            rec[L & 1].as<float4>(),
-                                           keys.as<uint32_t>(), prad, cnt, grid, n, s);
-                    if (e == hipSuccess && L < pp.max_depth) {
+                                           reorder ? keys.as<uint32_t>() : nullptr, prad, cnt, grid, n, s);
+                    if (e == hipSuccess && reorder && L < pp.max_depth) {
                         radix_sort_buffers rb{keys.as<uint32_t>(),      keys_tmp.as<uint32_t>(),
                                               vals_tmp.as<uint32_t>(),  perm.as<uint32_t>(),
                                               sort_counts.as<uint32_t>(), sort_totals.as<uint32_t>()};
@@ -704,6 +708,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
     HIP_TRY(p->frame_seed.alloc(8ull * samples));
     HIP_TRY(p->work.alloc(rt::dev::kCounterBytes));
     if (params->blocks <= 0) p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n, rt::dev::kGroupSlots8);
+    p->append_order = p->group && n <= rt::dev::kAppendSlots;
     p->pcfg.speculative = p->tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
     p->pcfg.refill = p->tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
     p->pcfg.refill_thr = params->refill_threshold > 0 ? std::min(params->refill_threshold, 64) : 40;

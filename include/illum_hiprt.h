@@ -281,7 +281,9 @@ typedef struct {
                                  widths): 0 = 4 + 28, 1 = 8 + 16, 2 = 2 + 20, 3 = 0 + 24,
                                  4 = 0 + 20 with registers capped for 8 waves per SIMD
                                  (binary trees, single scene); deeper traversals spill
-                                 to a global column per lane */
+                                 to a global column per lane.  Speculative any-hit and
+                                 batched launches over binary trees that need at most
+                                 32 entries hold the whole stack in LDS instead */
     int32_t work_chunks;      /* 1 = one work counter; 8 (and 0, the default) = one
                                  contiguous chunk of the rays per XCD, blocks start on
                                  their own XCD's chunk (fetch atomics spread over 8
@@ -490,8 +492,9 @@ int hiprt_integrate_light_sample(hiprt_scene sc, const hiprt_rays *cam_rays, con
  *                device, the whole frame captured once in a hipGraph.
  * In the batched schedule the queue of every bounce is, by default
  * (ray_order = 0), sorted by direction octant and origin cell (a 16^3 grid
- * over the scene box) so that wavefronts trace neighbouring rays; 1 keeps
- * the order the shading step appends them in.  Paths keep their own random
+ * over the scene box) so that wavefronts trace neighbouring rays; small frames,
+ * which several lanes per ray trace, are not sorted.  1 keeps the order the
+ * shading step appends them in.  Paths keep their own random
  * streams, so the image does not depend on the order.  samples > 1 traces
  * that many samples per pixel in one frame graph -- render call k traces the
  * samples of frames k*samples .. k*samples + samples - 1, with their own
