@@ -139,8 +139,14 @@ __global__ __launch_bounds__(256) void k_adjoint_vertices(adjoint_args a, const 
     }
 }
 
+// Small tiles while large ones are too few for the chip's 256 CUs.  Forward
+// and backward of the hall (three passes), us, tiles of 4096 / 1024: 131,072
+// rays 297 / 275, 262,144 430 / 408, 524,288 685 / 668, 1 M 1196 / 1188, 2 M
+// 3077 / 3076.
+static uint32_t sort_tile_of(uint32_t n) { return n <= 1u << 20 ? kSmallSortTile : kSortTile; }
+
 size_t adjoint_sort_bytes(uint32_t n) {
-    return 4ull * (13ull * n + 256ull * radix_tiles(n) + 256ull + 64ull);
+    return 4ull * (13ull * n + 256ull * radix_tiles(n, sort_tile_of(n)) + 256ull + 64ull);
 }
 
 hipError_t launch_adjoint_closest(const adjoint_args &a_in, uint32_t n, void *sort_scratch, hipStream_t s) {
@@ -151,7 +157,7 @@ hipError_t launch_adjoint_closest(const adjoint_args &a_in, uint32_t n, void *so
     if (vertices) {
         if (!sort_scratch) return hipErrorInvalidValue;
         uint32_t *w = static_cast<uint32_t *>(sort_scratch);
-        const uint32_t tiles = radix_tiles(n);
+        const uint32_t tiles = radix_tiles(n, sort_tile_of(n));
         rb.keys_in = w;
         rb.keys_tmp = w + n;
         rb.vals_tmp = w + 2ull * n;
@@ -167,7 +173,7 @@ hipError_t launch_adjoint_closest(const adjoint_args &a_in, uint32_t n, void *so
     if (e != hipSuccess || !vertices) return e;
     int bits = 1;
     while (bits < 32 && (a.n_tris >> bits) != 0u) ++bits;   // keys 0 .. n_tris
-    e = launch_radix_sort(rb, n, a.count, bits, s, true);   // the vertex pass reads the sorted keys
+    e = launch_radix_sort(rb, n, a.count, bits, s, true, sort_tile_of(n));   // the vertex pass reads the sorted keys
     if (e != hipSuccess) return e;
     // the last of the sort's passes leaves the keys in keys_tmp after an odd
     // number of passes, in keys_in after an even one

@@ -2,7 +2,7 @@
 // per pass, for the path tracer's bounce queues and the adjoint's triangle
 // keys.
 //
-// Per pass, over tiles of kSortTile consecutive items:
+// Per pass, over tiles of kSortTile (or kSmallSortTile) consecutive items:
 //   k_radix_count   digit histogram of each tile (LDS; one atomic for a wave
 //                   whose items share a digit), written digit-major
 //                   (counts[digit * n_tiles + tile]);
@@ -37,10 +37,9 @@ namespace {
 
 constexpr int kSortThreads = 256;
 constexpr int kSortWaves = kSortThreads / 64;
-constexpr int kSortRounds = kSortTile / kSortThreads;   // 64-item rounds in one wave's quarter of a tile
 constexpr int kDigits = 256;
 constexpr int kRowThreads = 1024;
-static_assert(kSortTile % kSortThreads == 0, "tile shape");
+static_assert(kSortTile % kSortThreads == 0 && kSmallSortTile % kSortThreads == 0, "tile shape");
 static_assert(kDigits == kSortThreads, "one thread per digit");
 
 // Tile of block b: XCD b mod 8 takes the b-th eighth of the tiles (the first
@@ -72,19 +71,21 @@ __device__ __forceinline__ uint64_t same_digit_lanes(uint32_t d, bool valid) {
     return same;
 }
 
+template <uint32_t TILE>
 __global__ __launch_bounds__(kSortThreads) void k_radix_count(const uint32_t *keys, const uint32_t *count_ptr,
                                                               uint32_t n_max, uint32_t shift, uint32_t dmask,
                                                               uint32_t *counts, uint32_t n_tiles) {
+    constexpr int kRounds = TILE / kSortThreads;
     __shared__ uint32_t hist[kDigits];
     const uint32_t n = min(*count_ptr, n_max);
     const uint32_t tile = sort_tile(blockIdx.x, n_tiles), t = threadIdx.x;
     hist[t] = 0u;
     __syncthreads();
-    const uint64_t first = (uint64_t)tile * kSortTile;
+    const uint64_t first = (uint64_t)tile * TILE;
     if (first < n) {   // every load in flight before the first atomic
-        uint32_t k[kSortRounds];
+        uint32_t k[kRounds];
 #pragma unroll
-        for (int s = 0; s < kSortRounds; ++s) {
+        for (int s = 0; s < kRounds; ++s) {
             const uint64_t i = first + (uint64_t)s * kSortThreads + t;
             k[s] = i < n ? keys[i] : 0u;
         }
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_count(const uint32_t *ke
         // passes, once lower digits have grouped the keys) adds once instead
         // of 64 times to the same LDS word
 #pragma unroll
-        for (int s = 0; s < kSortRounds; ++s) {
+        for (int s = 0; s < kRounds; ++s) {
             const bool valid = first + (uint64_t)s * kSortThreads + t < n;
             const uint32_t d = (k[s] >> shift) & dmask;
             const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
@@ -149,29 +150,31 @@ __global__ __launch_bounds__(kRowThreads) void k_radix_rows(uint32_t *counts, ui
     if (t == 0) totals[d] = carry;
 }
 
+template <uint32_t TILE>
 __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t *keys_in, const uint32_t *vals_in,
                                                                 const uint32_t *count_ptr, uint32_t n_max,
                                                                 uint32_t shift, uint32_t dmask,
                                                                 const uint32_t *counts, const uint32_t *totals,
                                                                 uint32_t n_tiles, uint32_t *keys_out,
                                                                 uint32_t *vals_out) {
-    constexpr uint32_t kQuarter = kSortTile / kSortWaves;
+    constexpr int kRounds = TILE / kSortThreads;   // 64-item rounds in one wave's quarter of a tile
+    constexpr uint32_t kQuarter = TILE / kSortWaves;
     __shared__ uint32_t slot[kDigits];              // queue slot of tile position 0 counted in each digit's run
     __shared__ uint32_t start[kDigits];             // tile position of each digit's first item
     __shared__ uint32_t wrun[kSortWaves][kDigits];  // items of each digit per wave, then the earlier waves' sum
     __shared__ uint32_t wsum[2][kSortWaves];
-    __shared__ uint32_t skey[kSortTile], sval[kSortTile];
+    __shared__ uint32_t skey[TILE], sval[TILE];
     const uint32_t n = min(*count_ptr, n_max);
     const uint32_t tile = sort_tile(blockIdx.x, n_tiles), t = threadIdx.x;
-    const uint64_t first = (uint64_t)tile * kSortTile;
+    const uint64_t first = (uint64_t)tile * TILE;
     if (first >= n) return;   // uniform: the whole tile is past the queue
     const uint32_t lane = t & 63u, wave = t >> 6;
 #pragma unroll
     for (int w = 0; w < kSortWaves; ++w) wrun[w][t] = 0u;
     const uint64_t quarter = first + (uint64_t)wave * kQuarter;
-    uint32_t key[kSortRounds], val[kSortRounds], loc[kSortRounds];
+    uint32_t key[kRounds], val[kRounds], loc[kRounds];
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         const uint64_t i = quarter + (uint64_t)r * 64u + lane;
         const bool valid = i < n;
         key[r] = valid ? keys_in[i] : 0u;
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t *
     // count) plus same-digit lanes below this one
     const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         const bool valid = quarter + (uint64_t)r * 64u + lane < n;
         const uint32_t d = (key[r] >> shift) & dmask;
         // one ballot settles a round whose valid lanes share a digit
@@ -226,7 +229,7 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t *
     slot[t] = pos_queue + counts[(size_t)t * n_tiles + tile] - pos_tile;   // mod 2^32; + a position >= start
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         if (quarter + (uint64_t)r * 64u + lane < n) {
             const uint32_t d = (key[r] >> shift) & dmask;
             const uint32_t p = start[d] + wrun[wave][d] + loc[r];
@@ -235,9 +238,9 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t *
         }
     }
     __syncthreads();
-    const uint32_t tn = (uint32_t)min((uint64_t)kSortTile, (uint64_t)n - first);
+    const uint32_t tn = (uint32_t)min((uint64_t)TILE, (uint64_t)n - first);
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
         const uint32_t j = (uint32_t)r * kSortThreads + t;
         if (j < tn) {
             const uint32_t k = skey[j];
@@ -252,11 +255,12 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const uint32_t *
 
 } // namespace
 
-uint32_t radix_tiles(uint32_t n_max) { return (uint32_t)(((uint64_t)n_max + kSortTile - 1) / kSortTile); }
+uint32_t radix_tiles(uint32_t n_max, uint32_t tile) { return (uint32_t)(((uint64_t)n_max + tile - 1) / tile); }
 
 hipError_t launch_radix_sort(const radix_sort_buffers &b, uint32_t n_max, const uint32_t *count_ptr, int bits,
-                             hipStream_t s, bool sorted_keys) {
-    const uint32_t tiles = radix_tiles(n_max);
+                             hipStream_t s, bool sorted_keys, uint32_t tile) {
+    if (tile != kSortTile && tile != kSmallSortTile) return hipErrorInvalidValue;
+    const uint32_t tiles = radix_tiles(n_max, tile);
     if (tiles == 0) return hipSuccess;
     const int passes = (bits + 7) / 8;
     if (passes < 1 || passes > 4) return hipErrorInvalidValue;
@@ -272,14 +276,16 @@ hipError_t launch_radix_sort(const radix_sort_buffers &b, uint32_t n_max, const 
         const uint32_t shift = 8u * (uint32_t)p;
         const int left = bits - 8 * p;   // key bits from `shift` on that take part
         const uint32_t dmask = left >= 8 ? 255u : (1u << left) - 1u;
-        hipLaunchKernelGGL(k_radix_count, dim3(tiles), dim3(kSortThreads), 0, s, kin, count_ptr, n_max, shift,
-                           dmask, b.counts, tiles);
+        const auto count = tile == kSortTile ? k_radix_count<kSortTile> : k_radix_count<kSmallSortTile>;
+        const auto scatter = tile == kSortTile ? k_radix_scatter<kSortTile> : k_radix_scatter<kSmallSortTile>;
+        hipLaunchKernelGGL(count, dim3(tiles), dim3(kSortThreads), 0, s, kin, count_ptr, n_max, shift, dmask,
+                           b.counts, tiles);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_radix_rows, dim3(kDigits), dim3(kRowThreads), 0, s, b.counts, tiles, b.totals);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_radix_scatter, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, count_ptr, n_max,
+        hipLaunchKernelGGL(scatter, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, count_ptr, n_max,
                            shift, dmask, b.counts, b.totals, tiles, kout, vout);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
