@@ -120,3 +120,30 @@ def test_opacity(torch_cuda, hip_ctx):
     ds = hiprt.DeviceScene(hip_ctx, sc, hiprt.Bvh(sc))
     _check(torch_cuda, ds, _rays(N, 31), tracer="while-while-alpha")
     ds.close()
+
+
+@pytest.mark.parametrize("tri", [hiprt.TRI_EXACT, hiprt.TRI_WOOP])
+def test_persistent_while_while_is_this_kernel(torch_cuda, hip_ctx, tri):
+    """Its own kernel, which a caller's grid selects, returns the same bits;
+    so does the allocation-free entry, in a tree that fits its stack and in
+    one that spills."""
+    torch = torch_cuda
+    pos, idx = nested_scene()
+    soup = hiprt.HostScene.random(3000, 0.06, 35)
+    deep = hiprt.HostScene.from_arrays(pos, idx)
+    for sc, max_tris, rays in ((soup, 4, _rays(N, 36)), (deep, 1, nested_rays(N, 37))):
+        ds = hiprt.DeviceScene(hip_ctx, sc, hiprt.Bvh(sc, max_tris=max_tris), hiprt.BVH2, tri)
+        dev = torch.from_numpy(rays).cuda()
+        want, got, free = (hiprt.new_hits(N) for _ in range(3))
+        hiprt.trace_closest(ds, dev, want, tracer="persistent-while-while", blocks=512)
+        hiprt.trace_closest(ds, dev, got, tracer="persistent-while-while")
+        hiprt.trace_closest_noalloc(ds, dev, free, blocks=512)
+        occ, occ2 = (torch.full((N,), 7, dtype=torch.uint8, device="cuda") for _ in range(2))
+        hiprt.trace_any(ds, dev, occ, tracer="persistent-while-while", blocks=512)
+        hiprt.trace_any(ds, dev, occ2, tracer="persistent-while-while")
+        torch.cuda.synchronize()
+        for k in got:
+            assert torch.equal(got[k].view(torch.int32), want[k].view(torch.int32)), k
+            assert torch.equal(free[k].view(torch.int32), want[k].view(torch.int32)), k
+        assert torch.equal(occ, occ2)
+        ds.close()
