@@ -36,14 +36,18 @@ class ClosestHit(torch.autograd.Function):
         hiprt.trace_closest(dscene, rays, hits, tracer=tracer)
         ctx.dscene = dscene
         ctx.n_vert = vertices.shape[0]
-        ctx.save_for_backward(rays, hits["t"], hits["u"], hits["v"], hits["id"])
+        # the adjoint recomputes u and v: only t and the ids are kept, apart
+        # from the returned tensors, which the caller may change in place
+        ctx.save_for_backward(rays, hits["t"], hits["id"])
+        # an output without a gradient comes as None: no zeros for tri
+        ctx.set_materialize_grads(False)
         tri = hits["id"].clone()
         ctx.mark_non_differentiable(tri)
-        return hits["t"].clone(), hits["u"].clone(), hits["v"].clone(), tri
+        return hits["t"].clone(), hits["u"], hits["v"], tri
 
     @staticmethod
     def backward(ctx, g_t, g_u, g_v, g_tri):
-        rays, t, u, v, tri = ctx.saved_tensors
+        rays, t, tri = ctx.saved_tensors
         n = rays.shape[1]
         dev = rays.device
         zeros = lambda: torch.zeros(n, dtype=torch.float32, device=dev)
@@ -53,7 +57,7 @@ class ClosestHit(torch.autograd.Function):
         gv = torch.zeros((ctx.n_vert, 3), dtype=torch.float32, device=dev)
         go = torch.empty((n, 3), dtype=torch.float32, device=dev)
         gd = torch.empty((n, 3), dtype=torch.float32, device=dev)
-        hits = {"t": t, "u": u, "v": v, "id": tri}
+        hits = {"t": t, "u": t, "v": t, "id": tri}   # u and v are not read
         hiprt.adjoint_closest(ctx.dscene, rays, hits, g_t, g_u, g_v, grad_vertices=gv, grad_origin=go, grad_dir=gd)
         return gv, go, gd, None, None
 
