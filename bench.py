@@ -83,7 +83,7 @@ def time_trace(torch, hiprt, ds, rays, tracer="dynamic-while-while", stream=None
 
 
 def kernel_name(kw, ds, binary):
-    """Template instantiation of the persistent closest-hit kernel that a
+    """Template instantiation of the closest-hit kernel that a large
     path-tracer configuration runs on scene `ds` (exact records)."""
     tracer = kw.get("tracer", "dynamic-while-while")
     spec = "true" if tracer in ("persistent-speculative-while-while", "dynamic-while-while") else "false"
@@ -93,6 +93,8 @@ def kernel_name(kw, ds, binary):
     # the LDS ring with a spill column when the tree outgrows the
     # configuration, the plain LDS stack otherwise
     ring = "true" if ds.stack_need > reg + lds else "false"
+    if spec == "true" and binary and ds.stack_need > 0:   # the stack in LDS, whatever the configuration
+        return f"k_trace_dynamic<0, false, false> ({tracer}, binary tree)"
     return (f"k_trace_persistent<0, false, {spec}, {refill}, {reg}, {lds}, false, {2 if binary else 4}, false, "
             f"{ring}> ({tracer}, stack {kw.get('stack_config', 0)}, {'binary' if binary else '4-wide'} tree)")
 
@@ -686,7 +688,7 @@ def main():
     d_pos = torch.from_numpy(pos).cuda()
     ms_refit = time_calls(torch, lambda: ds.refit(d_pos, stream.cuda_stream), stream, reps=10)
     ms_after, _ = time_trace(torch, hiprt, ds, d_diff, "dynamic-while-while", stream)
-    refit = {"ms": round(ms_refit, 4), "levels_launched": int(ds.depth),
+    refit = {"ms": round(ms_refit, 4), "tree_depth": int(ds.depth),
              "diffuse_after_refit_mrays": round(d_diff.shape[1] / ms_after / 1e3, 1)}
     log(f"refit: {refit}")
 

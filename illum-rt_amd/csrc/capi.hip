@@ -52,8 +52,9 @@ hipError_t attach_spill(hiprt_stream_state *st, hipStream_t s, const rt::scene_d
                         int need, rt::dev::persistent_cfg &cfg, int spill_limit) {
     cfg.spill = nullptr;
     cfg.need = spill_limit > 0 ? 0 : need;
-    if (rt::dev::dynamic_fits(d.bvh, any, multi, cfg)) return hipSuccess;   // its stack is in LDS
-    cfg.spill_cap = rt::dev::persistent_spill_entries(d.bvh, cfg.stack, need);
+    const bool lds = rt::dev::dynamic_fits(d.bvh, any, multi, cfg);
+    if (lds && (any || multi)) return hipSuccess;   // the whole stack is in LDS
+    cfg.spill_cap = lds ? rt::dev::dynamic_spill_entries(need) : rt::dev::persistent_spill_entries(d.bvh, cfg.stack, need);
     if (spill_limit > 0 && cfg.spill_cap > (uint32_t)spill_limit) cfg.spill_cap = (uint32_t)spill_limit;
     cfg.spill_bytes = 0;
     if (cfg.spill_cap == 0) return hipSuccess;

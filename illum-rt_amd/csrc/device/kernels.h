@@ -87,7 +87,7 @@ struct persistent_cfg {
     int32_t *spill = nullptr;
     uint32_t spill_cap = 0;
     size_t spill_bytes = 0;
-    int need = 0;         // the trees' stack need; 0: not known, or the caller bounds the spill column
+    int need = 0;         // the trees' stack need; 0: trace_persistent.hip's kernels (see dynamic_fits)
 };
 
 // `counter` points to kCounterBytes of device memory (cleared by the launch);
@@ -100,17 +100,20 @@ hipError_t launch_trace_persistent(const scene_desc &sc, const ray_soa &rays, co
                                    bool any, const persistent_cfg &cfg, hipStream_t stream,
                                    ray_gather gather = ray_gather{});
 
-// The postponing tracers of binary trees, with the tree's whole stack in LDS
-// (trace_dynamic.hip): any-hit of one scene, and descriptor tables.  Does a
-// launch of this kind take it?  Trees of more entries, launches that count
-// fetches and those whose caller bounds the spill column keep the kernels of
-// trace_persistent.hip, which call these.
+// The postponing tracers of binary trees, with the stack in LDS
+// (trace_dynamic.hip).  Does a launch of this kind take it?  cfg.need set to
+// 0 (the caller bounds the spill column, or must not depend on one), launches
+// that count fetches, and any-hit and table launches over trees of more than
+// kDynamicStackNeed entries keep the kernels of trace_persistent.hip, which
+// call these.  dynamic_spill_entries: cfg.spill_cap of a closest-hit launch of
+// one scene (0 when the stack fits); the others need no column.
 constexpr int kDynamicStackNeed = 32;
 bool dynamic_fits(int bvh, bool any, bool multi, const persistent_cfg &cfg);
+uint32_t dynamic_spill_entries(int need);
 hipError_t dynamic_grid(int tri, bool any, bool multi, const persistent_cfg &cfg, int *blocks);
 hipError_t launch_trace_dynamic(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,
-                                uint32_t n, const uint32_t *count_ptr, uint32_t *counter, const persistent_cfg &cfg,
-                                hipStream_t stream, ray_gather gather);
+                                uint32_t n, const uint32_t *count_ptr, uint32_t *counter, bool any,
+                                const persistent_cfg &cfg, hipStream_t stream, ray_gather gather);
 hipError_t launch_trace_dynamic_batch(const batch_desc *d_table, uint32_t n_desc, uint32_t total, int tri, bool any,
                                       uint32_t *counter, const persistent_cfg &cfg, hipStream_t stream);
 

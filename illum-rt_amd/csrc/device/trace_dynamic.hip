@@ -1,34 +1,40 @@
-// Postponing persistent trace of binary trees with the whole traversal stack
-// in LDS: any-hit of the speculative tracers, and descriptor tables.
+// Postponing persistent trace of binary trees with the traversal stack in
+// LDS: the speculative tracers' closest and any hits of one scene, and
+// descriptor tables.
 //
 // The work and its order are trace_persistent.hip's (parked leaves, a vote
 // that ends the node loop, refill from the work counters): what differs is
 // how a lane's step is written.
-//   * Tree and ray bound the stack (the tree's stack need, at most
-//     kDynamicStackNeed), so it is an LDS column of that many words and two
-//     sentinels below: no overflow test, no empty test, no spill column.
+//   * Tree and ray bound the stack (the tree's stack need), so it is an LDS
+//     column with two sentinels below and no empty test.  Any-hit and table
+//     launches hold all of it (at most kDynamicStackNeed entries) and need no
+//     overflow test either.  Closest hits of one scene keep kSpillWords words,
+//     which leaves room for 7 waves per SIMD: a push on a full column moves
+//     the kSpillStep oldest entries to a global column per lane, and a lane
+//     that runs into the sentinel fetches them back once per leaf phase.
 //   * The two newest entries are read before the node arrives.  A miss, a
 //     hit, a parked leaf and a pop are then selects between registers, where
 //     the other kernel branches and waits for LDS after the box tests.
 //   * All control flow outside the step is wave-uniform, and ended rays are
 //     written when the wavefront leaves to take new ones; a closest hit's
 //     barycentrics are computed again there.  60 VGPRs (any-hit, single
-//     scene) and 74 (closest hit, table).
+//     scene), 71 (closest) and 74 (closest, table).
 //
-// Bound: address and cache-line rate of the node fetches (64 lanes, 64
-// lines) on incoherent rays, VALU issue and idle lanes on coherent ones.
+// Bound: VALU issue (99% of it on 8.3 M bounce rays, at 32% of the lanes) and
+// L1 (1.05 line accesses a clock there) at once; on camera rays VALU alone.
 // Measured, trace_persistent's kernel (its fastest stack configuration for
-// single scenes) -> this one: any-hit dynamic, hall, 2.07 M camera rays 1160
-// -> 1075 us, bounce 1885 -> 1735, random 1950 -> 1850, 8.3 M rays 3065 ->
-// 3015, 5770 -> 5530, 6670 -> 6510; persistent-speculative 2.07 M 1165 ->
-// 1078, 2205 -> 2140, 2150 -> 2105; soup 2.07 M 327 -> 307, 385 -> 343, 793
-// -> 760.  Descriptor tables, closest hit, random rays: 24 scenes x 200 k
-// rays of 5 k triangles 2355 -> 1985 (speculative), 1765 -> 1615 (dynamic);
-// 8 x 500 k of 90 k 3630 -> 2970, 2575 -> 2400; 3 x 1.1 M of 250 k 3440 ->
-// 2860, 2545 -> 2400.  Closest hit of one scene stays with trace_persistent,
-// whose 20 LDS words leave room for 8 waves per SIMD: 8.3 M bounce rays 5340
-// there, 5840 here (1030 against 980 at 921 k, 1133 against 1040 for 2.07 M
-// camera rays: what is won there is lost on larger incoherent batches).
+// single scenes) -> this one, us.  Closest hit, dynamic tracer, hall camera /
+// bounce / random rays: 921 k 733 -> 657, 1036 -> 956, 1026 -> 950; 2.07 M
+// 1118 -> 1018, 1699 -> 1628, 1782 -> 1750; 8.3 M 3103 -> 3023, 5325 -> 5329,
+// 6175 -> 6166 (persistent-speculative 2935 -> 2860, 6406 -> 6283, 7089 ->
+// 7060); soup 2.07 M 333 -> 305, 393 -> 353, 809 -> 784.  The whole 24 words
+// in LDS: 8.3 M random 7480 (6 waves per SIMD); registers capped for 8 waves:
+// bounce 5405, 921 k 1036.  Any-hit, dynamic tracer: hall 2.07 M 1160 -> 1075,
+// 1885 -> 1735, 1950 -> 1850, 8.3 M 3065 -> 3015, 5770 -> 5530, 6670 -> 6510;
+// soup 327 -> 307, 385 -> 343, 793 -> 760.  Descriptor tables, closest hit,
+// random rays: 24 scenes x 200 k rays of 5 k triangles 2355 -> 1985
+// (speculative), 1765 -> 1615 (dynamic); 8 x 500 k of 90 k 3630 -> 2970, 2575
+// -> 2400; 3 x 1.1 M of 250 k 3440 -> 2860, 2545 -> 2400.
 #include "kernels.h"
 #include "trace_core.h"
 
@@ -48,15 +54,21 @@ struct dynamic_args {
     const batch_desc *table;
     uint32_t n_desc;
     ray_gather gather;
-    uint32_t entries;   // LDS words per lane: two sentinels and the stack need
+    uint32_t entries;   // LDS words per lane: two sentinels and the stack need, or as much of it as fits
+    int32_t *spill;     // columns of the oldest entries, one per lane (closest hits of one scene)
     uint32_t chunks;
     int32_t refill_thr, park;
 };
 
+// Closest hits of one scene: LDS words per lane, sentinels included, and the
+// entries that move between them and the global column at a time.
+constexpr uint32_t kSpillWords = 20;
+constexpr int kSpillStep = 4;
+
 } // namespace
 
 template <int TRI, bool ANY, bool MULTI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 7 : 6)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ANY ? 7 : MULTI ? 6 : 7)))
 void k_trace_dynamic(dynamic_args a) {
     extern __shared__ int32_t lds_words[];
     const uint32_t n = a.count_ptr ? *a.count_ptr : a.n;
@@ -64,6 +76,9 @@ void k_trace_dynamic(dynamic_args a) {
     int32_t *col = lds_words + (threadIdx.x >> 6) * 64u * a.entries + lane;
     col[0] = kInvalidRef;
     col[64] = kInvalidRef;
+    constexpr bool SPILL = !ANY && !MULTI;
+    const int top = (int)(64u * a.entries);   // sp when the LDS part is full
+    int gs = 0;                               // entries moved to the global column
     uint32_t chunk = blockIdx.x % a.chunks, dry = 0;
     bool exhausted = false, alive = false, finite = true;
     const char *nodes = static_cast<const char *>(a.sc.nodes);
@@ -126,6 +141,7 @@ void k_trace_dynamic(dynamic_args a) {
                     finite = nan_free && ray_is_finite(r);
                     cur = root;
                     sp = 128;
+                    gs = 0;
                     pc = 0;
                     found = false;
                     ht = ANY ? INFINITY : FLT_MAX;
@@ -166,7 +182,17 @@ void k_trace_dynamic(dynamic_args a) {
                         any = hl || hr;
                         const bool left = hl && (!hr || dl < dr);
                         const int32_t far_ref = left ? rr : rl;
-                        if (both) col[sp] = far_ref;
+                        if (both) {
+                            if (SPILL && sp == top) {   // rare: the oldest entries go to the global column
+                                int32_t *g = a.spill + blockIdx.x * 256u + threadIdx.x;
+                                const size_t stride = gridDim.x * 256u;
+                                for (int k = 0; k < kSpillStep; ++k) g[(gs + k) * stride] = col[64 * (2 + k)];
+                                gs += kSpillStep;
+                                for (int k = 128; k < top - 64 * kSpillStep; k += 64) col[k] = col[k + 64 * kSpillStep];
+                                sp -= 64 * kSpillStep;
+                            }
+                            col[sp] = far_ref;
+                        }
                         c = any ? (left ? rl : rr) : t0;
                         next = both ? far_ref : (any ? t0 : t1);
                         d = both ? 64 : (any ? 0 : -64);
@@ -217,6 +243,14 @@ void k_trace_dynamic(dynamic_args a) {
                     pc = 0;
                     break;
                 }
+            }
+            if (SPILL && cur == kInvalidRef && gs > 0) {   // the LDS part is empty: the column's newest entries
+                int32_t *g = a.spill + blockIdx.x * 256u + threadIdx.x;
+                const size_t stride = gridDim.x * 256u;
+                gs -= kSpillStep;
+                for (int k = 0; k < kSpillStep; ++k) col[64 * (2 + k)] = g[(gs + k) * stride];
+                sp = 64 * (kSpillStep + 1);
+                cur = col[sp];
             }
         } while (exhausted ? wave_mask(cur != kInvalidRef) != 0
                            : (int)__popcll(wave_mask(cur != kInvalidRef)) >= a.refill_thr);
@@ -295,16 +329,23 @@ hipError_t launch_one(const dynamic_args &a, const persistent_cfg &cfg, hipStrea
         *grid_out = blocks;
         return hipSuccess;
     }
+    const uint32_t column = ANY || MULTI ? 0u : dynamic_spill_entries(cfg.need);
+    if (column && (!cfg.spill || cfg.spill_bytes < persistent_spill_bytes(blocks, column))) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_trace_dynamic<TRI, ANY, MULTI>), dim3(blocks), dim3(256), 1024u * a.entries, s, a);
     return hipGetLastError();
 }
 
 hipError_t dispatch(int tri, bool any, bool multi, dynamic_args &a, const persistent_cfg &cfg, hipStream_t s,
                     int *grid_out) {
-    a.entries = (uint32_t)cfg.need + kSentinels;
+    a.entries = any || multi ? (uint32_t)cfg.need + kSentinels
+                             : min((uint32_t)cfg.need + kSentinels, kSpillWords);
+    a.spill = cfg.spill;
     a.chunks = cfg.chunks == 8 ? 8u : 1u;
     a.refill_thr = cfg.refill ? (cfg.refill_thr < 1 ? 1 : (cfg.refill_thr > 64 ? 64 : cfg.refill_thr)) : 1;
     a.park = cfg.park < 1 || cfg.park > kParkClosest ? kParkClosest : cfg.park;
+    if (!multi && !any)
+        return tri == TRI_EXACT ? launch_one<TRI_EXACT, false, false>(a, cfg, s, grid_out)
+                                : launch_one<TRI_WOOP, false, false>(a, cfg, s, grid_out);
     if (!multi)
         return tri == TRI_EXACT ? launch_one<TRI_EXACT, true, false>(a, cfg, s, grid_out)
                                 : launch_one<TRI_WOOP, true, false>(a, cfg, s, grid_out);
@@ -317,9 +358,14 @@ hipError_t dispatch(int tri, bool any, bool multi, dynamic_args &a, const persis
 
 } // namespace
 
+uint32_t dynamic_spill_entries(int need) {
+    const int over = need - (int)(kSpillWords - kSentinels);
+    return over > 0 ? (uint32_t)((over + kSpillStep - 1) / kSpillStep * kSpillStep) : 0u;
+}
+
 bool dynamic_fits(int bvh, bool any, bool multi, const persistent_cfg &cfg) {
-    return (any || multi) && bvh == BVH2 && cfg.speculative && !cfg.stats && cfg.need > 0 &&
-           cfg.need <= kDynamicStackNeed;
+    return bvh == BVH2 && cfg.speculative && !cfg.stats && cfg.need > 0 &&
+           (cfg.need <= kDynamicStackNeed || !(any || multi));
 }
 
 hipError_t dynamic_grid(int tri, bool any, bool multi, const persistent_cfg &cfg, int *blocks) {
@@ -328,8 +374,8 @@ hipError_t dynamic_grid(int tri, bool any, bool multi, const persistent_cfg &cfg
 }
 
 hipError_t launch_trace_dynamic(const scene_desc &sc, const ray_soa &rays, const hit_soa &hits, uint8_t *occluded,
-                                uint32_t n, const uint32_t *count_ptr, uint32_t *counter, const persistent_cfg &cfg,
-                                hipStream_t stream, ray_gather gather) {
+                                uint32_t n, const uint32_t *count_ptr, uint32_t *counter, bool any,
+                                const persistent_cfg &cfg, hipStream_t stream, ray_gather gather) {
     dynamic_args a{};
     a.sc = sc;
     a.rays = rays;
@@ -339,7 +385,7 @@ hipError_t launch_trace_dynamic(const scene_desc &sc, const ray_soa &rays, const
     a.count_ptr = count_ptr;
     a.counter = counter;
     a.gather = gather;
-    return dispatch(sc.tri, true, false, a, cfg, stream, nullptr);
+    return dispatch(sc.tri, any, false, a, cfg, stream, nullptr);
 }
 
 hipError_t launch_trace_dynamic_batch(const batch_desc *d_table, uint32_t n_desc, uint32_t total, int tri, bool any,

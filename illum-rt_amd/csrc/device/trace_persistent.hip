@@ -625,7 +625,7 @@ hipError_t launch_trace_persistent(const scene_desc &sc, const ray_soa &rays, co
     hipError_t e = launch_fill_u32(counter, 0u, kMaxChunks * kCounterStride, stream);
     if (e != hipSuccess) return e;
     if (dynamic_fits(sc.bvh, any, false, cfg))
-        return launch_trace_dynamic(sc, rays, hits, occluded, n, count_ptr, counter, cfg, stream, gather);
+        return launch_trace_dynamic(sc, rays, hits, occluded, n, count_ptr, counter, any, cfg, stream, gather);
     launch_args a{sc, rays, gather, hits, occluded, n, count_ptr, counter, nullptr, 0};
     return dispatch<false>(sc.tri, any, sc.bvh, a, cfg, stream, false, nullptr);
 }

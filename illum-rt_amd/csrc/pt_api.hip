@@ -730,13 +730,16 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
         HIP_TRY(grid_of(sc, &p->grid));
     }
     if (p->batched) {
+        p->pcfg.need = sc->stack_need;
         // Resolve the persistent grid size outside the capture, then record
         // the frame once.  The graph never clears the accumulator: frame 0
         // after a reset is rendered eagerly with clear_radiance set.
         if (params->blocks > 0) p->pcfg.blocks = params->blocks;
         else HIP_TRY(rt::dev::persistent_grid(sc->desc, false, p->pcfg, &p->pcfg.blocks));
         // the graph keeps the spill buffer's address: allocate it for the grid now
-        p->pcfg.spill_cap = rt::dev::persistent_spill_entries(sc->desc.bvh, stack, sc->stack_need);
+        p->pcfg.spill_cap = rt::dev::dynamic_fits(sc->desc.bvh, false, false, p->pcfg)
+                                ? rt::dev::dynamic_spill_entries(sc->stack_need)
+                                : rt::dev::persistent_spill_entries(sc->desc.bvh, stack, sc->stack_need);
         if (p->pcfg.spill_cap) {
             HIP_TRY(p->spill.alloc(rt::dev::persistent_spill_bytes(p->pcfg.blocks, p->pcfg.spill_cap)));
             p->pcfg.spill = p->spill.as<int32_t>();

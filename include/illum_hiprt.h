@@ -281,9 +281,11 @@ typedef struct {
                                  widths): 0 = 4 + 28, 1 = 8 + 16, 2 = 2 + 20, 3 = 0 + 24,
                                  4 = 0 + 20 with registers capped for 8 waves per SIMD
                                  (binary trees, single scene); deeper traversals spill
-                                 to a global column per lane.  Speculative any-hit and
-                                 batched launches over binary trees that need at most
-                                 32 entries hold the whole stack in LDS instead */
+                                 to a global column per lane.  Speculative launches over
+                                 binary trees hold their stack in LDS whatever the
+                                 configuration, unless they count fetches, bound the
+                                 spill column or must not allocate (any-hit and batches:
+                                 or the tree needs more than 32 entries) */
     int32_t work_chunks;      /* 1 = one work counter; 8 (and 0, the default) = one
                                  contiguous chunk of the rays per XCD, blocks start on
                                  their own XCD's chunk (fetch atomics spread over 8

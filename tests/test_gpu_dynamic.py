@@ -1,6 +1,6 @@
-"""The postponing kernel with its stack in LDS (any-hit of one scene, and
-descriptor tables) against the oracle: wavefront remainders, refill
-thresholds, work counters, triangle formats, opacity, rays with non-finite
+"""The postponing kernel with its stack in LDS (one scene, and descriptor
+tables) against the oracle: wavefront remainders, refill thresholds, work
+counters, parked leaves, triangle formats, opacity, rays with non-finite
 components, trees just inside and outside of its stack, a scene that is one
 leaf.  A caller's grid selects the kernel at any size; occlusion is compared
 exactly, closest hits up to ties."""
@@ -89,6 +89,56 @@ def test_stack_of_the_tree(torch_cuda, hip_ctx, limit):
                                            spill_limit=limit), want)
         ds.close()
     assert min(needs) < 32 < max(needs), needs
+
+
+def _closest(torch, ds, rays, **kw):
+    h = hiprt.new_hits(rays.shape[1])
+    for x in h.values():
+        x.fill_(-5)
+    hiprt.trace_closest(ds, torch.from_numpy(rays).cuda(), h, **kw)
+    torch.cuda.synchronize()
+    return tuple(h[k].cpu().numpy() for k in ("t", "u", "v")) + (h["id"].cpu().numpy().view(np.uint32),)
+
+
+@pytest.mark.parametrize("tracer", SPEC)
+@pytest.mark.parametrize("n", [1, 64, 257, 30001])
+@pytest.mark.parametrize("blocks,refill,chunks,park", [(1, 1, 8, 1), (3, 40, 8, 2), (3, 64, 1, 3), (200, 0, 0, 4)])
+def test_closest_hit(torch_cuda, hip_ctx, soup, tracer, n, blocks, refill, chunks, park):
+    print(f"case: closest hit, {n} rays, {tracer}, {blocks} blocks, {park} parked leaves", flush=True)
+    sc, bvh = soup
+    pos, idx, _ = sc.arrays()
+    rays = _rays(n, n)
+    want = orc.trace_closest(pos, idx, bvh.nodes, bvh.root, bvh.index, rays)
+    ds = hiprt.DeviceScene(hip_ctx, sc, bvh)
+    got = _closest(torch_cuda, ds, rays, tracer=tracer, blocks=blocks, refill_threshold=refill, work_chunks=chunks,
+                   park_leaves=park)
+    assert classify(orc, pos, idx, rays, got, want)["unexplained"] == 0
+    ds.close()
+
+
+@pytest.mark.parametrize("tri", [hiprt.TRI_EXACT, hiprt.TRI_WOOP])
+def test_closest_hit_columns(torch_cuda, hip_ctx, tri):
+    """Trees whose stack fits the LDS words and trees that spill one group of
+    entries and more: the counting kernel, with a stack of its own, finds the
+    same hits."""
+    torch = torch_cuda
+    needs = set()
+    for n_tris in (12, 55, 60, 65, 75, 90, 105, 120):
+        pos, idx = nested_scene()
+        pos, idx = np.ascontiguousarray(pos[:3 * n_tris]), np.ascontiguousarray(idx[:n_tris])
+        sc = hiprt.HostScene.from_arrays(pos, idx)
+        ds = hiprt.DeviceScene(hip_ctx, sc, hiprt.Bvh(sc, max_tris=1), hiprt.BVH2, tri)
+        print(f"case: {n_tris} nested triangles, stack need {ds.stack_need}", flush=True)
+        needs.add(ds.stack_need)
+        rays = nested_rays(20000, n_tris)
+        stats = torch.zeros(2, dtype=torch.int64, device="cuda")
+        want = _closest(torch, ds, rays, fetch_stats=stats)
+        for tracer in SPEC:
+            for blocks in (2, 300):
+                got = _closest(torch, ds, rays, tracer=tracer, blocks=blocks)
+                assert classify(orc, pos, idx, rays, got, want)["unexplained"] == 0, (tracer, blocks)
+        ds.close()
+    assert min(needs) < 18 < max(needs), needs
 
 
 def _scenes(hip_ctx, tri):
