@@ -15,10 +15,11 @@
 //   * The two newest entries are read before the node arrives.  A miss, a
 //     hit, a parked leaf and a pop are then selects between registers, where
 //     the other kernel branches and waits for LDS after the box tests.
-//   * All control flow outside the step is wave-uniform, and ended rays are
-//     written when the wavefront leaves to take new ones; a closest hit's
-//     barycentrics are computed again there.  60 VGPRs (any-hit, single
-//     scene), 71 (closest) and 74 (closest, table).
+//   * All control flow outside the step is wave-uniform.  Closest hits are
+//     written when the wavefront leaves to take new rays, with barycentrics
+//     computed again there (each leaf phase: 2-3% slower); any-hit results
+//     after each leaf phase (8.3 M random rays 5635 us, when it leaves 6496).
+//     70 VGPRs (any-hit), 71 (closest) and 74 (closest, table).
 //
 // Bound: VALU issue (99% of it on 8.3 M bounce rays, at 32% of the lanes) and
 // L1 (1.05 line accesses a clock there) at once; on camera rays VALU alone.
@@ -30,8 +31,8 @@
 // 7060); soup 2.07 M 333 -> 305, 393 -> 353, 809 -> 784.  The whole 24 words
 // in LDS: 8.3 M random 7480 (6 waves per SIMD); registers capped for 8 waves:
 // bounce 5405, 921 k 1036.  Any-hit, dynamic tracer: hall 2.07 M 1160 -> 1075,
-// 1885 -> 1735, 1950 -> 1850, 8.3 M 3065 -> 3015, 5770 -> 5530, 6670 -> 6510;
-// soup 327 -> 307, 385 -> 343, 793 -> 760.  Descriptor tables, closest hit,
+// 1885 -> 1690, 1950 -> 1658, 8.3 M 3065 -> 3000, 5770 -> 5350, 6670 -> 5635;
+// soup 327 -> 302, 385 -> 339, 793 -> 739.  Descriptor tables, closest hit,
 // random rays: 24 scenes x 200 k rays of 5 k triangles 2355 -> 1985
 // (speculative), 1765 -> 1615 (dynamic); 8 x 500 k of 90 k 3630 -> 2970, 2575
 // -> 2400; 3 x 1.1 M of 250 k 3440 -> 2860, 2545 -> 2400.
@@ -96,6 +97,35 @@ void k_trace_dynamic(dynamic_args a) {
     uint32_t hslot = 0;
     bool found = false;
     bool exact = false;
+
+    // ---- ended rays: write the result, the lane is idle ----
+    auto end_rays = [&]() {
+        if (alive && cur == kInvalidRef) {
+            hit_soa ho = a.hits;
+            uint8_t *occ = a.occluded;
+            if (MULTI) {
+                ho = a.table[desc].hits;
+                occ = a.table[desc].occluded;
+            }
+            if (ANY) {
+                if (occ) occ[ray_id] = found ? 1 : 0;
+                if (ho.t)
+                    store_hit(ho, ray_id, found ? 4294967295.0f : FLT_MAX, 0.0f, 0.0f, found ? 0xffffffffu : 0u);
+            } else if (found) {
+                // the hit's barycentrics, by the same arithmetic again: two
+                // registers less to carry
+                const float4 *p = reinterpret_cast<const float4 *>(tris + hslot);
+                float4 r0 = p[0], r1 = p[1], r2 = p[2];
+                float t = ht, u = 0.0f, v = 0.0f;
+                if (TRI == TRI_EXACT) (void)tri_exact(r0, r1, r2, r, INFINITY, t, u, v);
+                else (void)tri_woop(r0, r1, r2, r, INFINITY, t, u, v);
+                store_hit(ho, ray_id, t, u, v, TRI == TRI_EXACT ? __float_as_uint(r0.w) : slot_ids[hslot]);
+            } else {
+                store_hit(ho, ray_id, FLT_MAX, 0.0f, 0.0f, 0u);
+            }
+            alive = false;
+        }
+    };
 
     for (;;) {
         // ---- idle lanes take new rays: one atomic per wavefront ----
@@ -252,34 +282,10 @@ void k_trace_dynamic(dynamic_args a) {
                 sp = 64 * (kSpillStep + 1);
                 cur = col[sp];
             }
+            if (ANY) end_rays();
         } while (exhausted ? wave_mask(cur != kInvalidRef) != 0
                            : (int)__popcll(wave_mask(cur != kInvalidRef)) >= a.refill_thr);
-        // ---- ended rays ----
-        if (alive && cur == kInvalidRef) {
-            hit_soa ho = a.hits;
-            uint8_t *occ = a.occluded;
-            if (MULTI) {
-                ho = a.table[desc].hits;
-                occ = a.table[desc].occluded;
-            }
-            if (ANY) {
-                if (occ) occ[ray_id] = found ? 1 : 0;
-                if (ho.t)
-                    store_hit(ho, ray_id, found ? 4294967295.0f : FLT_MAX, 0.0f, 0.0f, found ? 0xffffffffu : 0u);
-            } else if (found) {
-                // the hit's barycentrics, by the same arithmetic again: two
-                // registers less to carry
-                const float4 *p = reinterpret_cast<const float4 *>(tris + hslot);
-                float4 r0 = p[0], r1 = p[1], r2 = p[2];
-                float t = ht, u = 0.0f, v = 0.0f;
-                if (TRI == TRI_EXACT) (void)tri_exact(r0, r1, r2, r, INFINITY, t, u, v);
-                else (void)tri_woop(r0, r1, r2, r, INFINITY, t, u, v);
-                store_hit(ho, ray_id, t, u, v, TRI == TRI_EXACT ? __float_as_uint(r0.w) : slot_ids[hslot]);
-            } else {
-                store_hit(ho, ray_id, FLT_MAX, 0.0f, 0.0f, 0u);
-            }
-            alive = false;
-        }
+        if (!ANY) end_rays();
         if (exhausted) break;
     }
 }
@@ -294,8 +300,8 @@ constexpr uint32_t kSentinels = 2;
 // take 4 blocks per CU (16 wavefronts) when more fit: their 64 rays are the
 // least alike, and more wavefronts evict each other's nodes (3 x 1.1 M rays
 // of 250 k triangles: 6 blocks 2745 us, 5 2620, 4 2395; 24 x 200 k of 5 k
-// 1580, 1560, 1615).  Any-hit keeps all: 8.3 M random rays 6513 us with 6
-// blocks, 5973 with 4, but camera rays 3012 and 3451.
+// 1580, 1560, 1615).  Any-hit keeps all: camera rays, 8.3 M, 3012 us with 6
+// blocks, 3451 with 4.
 template <int TRI, bool ANY, bool MULTI>
 hipError_t grid_of(uint32_t entries, bool refill, int *blocks) {
     static int cached[64][kDynamicStackNeed + kSentinels + 1] = {};
