@@ -473,18 +473,42 @@ std::string check_layout(rt::flat_scene &f, uint32_t &stack_need) {
     return "";
 }
 
-// Does every child's box hold the boxes stored in that child?  (NaN: no.)
-static bool boxes_nested(const std::vector<rt::node2> &nodes) {
-    auto inside = [](const rt::node2 &c, float xlo, float xhi, float ylo, float yhi, float zlo, float zhi) {
-        return c.lxlo >= xlo && c.lxhi <= xhi && c.lxlo <= c.lxhi && c.rxlo >= xlo && c.rxhi <= xhi && c.rxlo <= c.rxhi &&
-               c.lylo >= ylo && c.lyhi <= yhi && c.lylo <= c.lyhi && c.rylo >= ylo && c.ryhi <= yhi && c.rylo <= c.ryhi &&
-               c.lzlo >= zlo && c.lzhi <= zhi && c.lzlo <= c.lzhi && c.rzlo >= zlo && c.rzhi <= zhi && c.rzlo <= c.rzhi;
-    };
-    for (const rt::node2 &n : nodes) {
-        if (!rt::ref_is_leaf(n.ref_l) && !inside(nodes[n.ref_l], n.lxlo, n.lxhi, n.lylo, n.lyhi, n.lzlo, n.lzhi)) return false;
-        if (!rt::ref_is_leaf(n.ref_r) && !inside(nodes[n.ref_r], n.rxlo, n.rxhi, n.rylo, n.ryhi, n.rzlo, n.rzhi)) return false;
+// One pass over the nodes, four bounds at a time: is no box bound NaN, and
+// (binary trees) does every child's box hold the boxes stored in that child,
+// none of them inverted?  Bounds of absent 4-wide children are +-inf, never
+// NaN.  A NaN bound answers no to both.
+typedef float float_x4 __attribute__((vector_size(16)));
+typedef int int_x4 __attribute__((vector_size(16)));
+
+static void check_boxes(const rt::flat_scene &h, bool &nan_free, bool &nested) {
+    const bool binary = h.bvh_kind == rt::BVH2;
+    const size_t n = binary ? h.nodes2.size() : h.nodes4.size();
+    const float_x4 *f = binary ? reinterpret_cast<const float_x4 *>(h.nodes2.data())
+                               : reinterpret_cast<const float_x4 *>(h.nodes4.data());
+    const int row = binary ? 4 : 8, boxes = binary ? 3 : 6;
+    int_x4 nan = {}, out = {};
+    for (size_t i = 0; i < n * row; i += row)
+        for (int k = 0; k < boxes; ++k) nan |= f[i + k] != f[i + k];
+    if (binary) {
+        const float_x4 sign = {1.0f, -1.0f, 1.0f, -1.0f};   // (lo, -hi): inside is >= in every place
+        for (size_t i = 0; i < n; ++i) {
+            const float_x4 *p = f + 4 * i;
+            const float_x4 l = p[0] * sign, r = p[1] * sign, z = p[2] * sign;
+            const float_x4 lz = __builtin_shufflevector(z, z, 0, 1, 0, 1), rz = __builtin_shufflevector(z, z, 2, 3, 2, 3);
+            const float_x4 lo = __builtin_shufflevector(l, r, 0, 2, 4, 6), hi = __builtin_shufflevector(l, r, 1, 3, 5, 7);
+            out |= ~(lo <= -hi) | ~(lz <= -__builtin_shufflevector(lz, lz, 1, 0, 1, 0)) |
+                   ~(rz <= -__builtin_shufflevector(rz, rz, 1, 0, 1, 0));
+            for (int k = 0; k < 2; ++k) {
+                const int32_t ref = k ? h.nodes2[i].ref_r : h.nodes2[i].ref_l;
+                if (rt::ref_is_leaf(ref)) continue;
+                const float_x4 *c = f + 4 * (size_t)ref;
+                const float_x4 xy = k ? r : l, zz = __builtin_shufflevector(k ? rz : lz, z, 0, 1, 0, 1);
+                out |= ~(c[0] * sign >= xy) | ~(c[1] * sign >= xy) | ~(c[2] * sign >= zz);
+            }
+        }
     }
-    return true;
+    nan_free = (nan[0] | nan[1] | nan[2] | nan[3]) == 0;
+    nested = binary && (out[0] | out[1] | out[2] | out[3]) == 0;
 }
 
 void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
@@ -499,18 +523,10 @@ void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
     s->stack_need = (int)stack_need;
     s->n_nodes = (uint32_t)(h.bvh_kind == rt::BVH2 ? h.nodes2.size() : h.nodes4.size());
     s->n_slots = (uint32_t)h.tris.size();
-    {
-        // box bounds of absent 4-wide children are +-inf, never NaN
-        const float *fv = h.bvh_kind == rt::BVH2 ? reinterpret_cast<const float *>(h.nodes2.data())
-                                                 : reinterpret_cast<const float *>(h.nodes4.data());
-        size_t nf = h.bvh_kind == rt::BVH2 ? h.nodes2.size() * 16 : h.nodes4.size() * 32;
-        size_t row = h.bvh_kind == rt::BVH2 ? 16 : 32, boxes = h.bvh_kind == rt::BVH2 ? 12 : 24;
-        bool nan_free = true;
-        for (size_t k = 0; k < nf && nan_free; ++k)
-            if (k % row < boxes && std::isnan(fv[k])) nan_free = false;
-        s->desc.nan_free = nan_free ? 1 : 0;
-    }
-    s->desc.nested = h.bvh_kind == rt::BVH2 && boxes_nested(h.nodes2) ? 1 : 0;
+    bool nan_free = true, nested = false;
+    check_boxes(h, nan_free, nested);
+    s->desc.nan_free = nan_free ? 1 : 0;
+    s->desc.nested = nested ? 1 : 0;
 }
 
 hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
