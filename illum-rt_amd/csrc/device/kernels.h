@@ -137,19 +137,19 @@ hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg 
 // and persistent kernels serve those.  Hall, us, camera / bounce rays:
 //   16 -> 8: 320 x 240 (77k) 124 / 131 against 129 / 139, but 53 / 41 against
 //   43 / 44 in the 8,192-triangle scene.
-//   8 -> 0: 800 x 600 (480k) 496 / 526, plain 631 / 851, dynamic 699 / 855;
-//   1281 x 719 (921k) 832 / 910, plain 787 / 1220, dynamic 723 / 1027 (any
-//   hit 730 / 781, plain 784 / 1191, dynamic 805 / 1191);
-//   1920 x 1080 (2.07M) 1734 / 1912, plain 1250 / 2262, dynamic 1118 / 1678.
+//   8 -> 0: 960 x 540 (518k) 504 / 547, plain 576 / 789; 1280 x 720 (922k)
+//   839 / 913, plain 740 / 1128, dynamic 657 / 956 (any hit 748 / 793, plain
+//   695 / 1201); 1920 x 1080 (2.07M) 1734 / 1912, plain
+//   1181 / 2069, dynamic 1018 / 1628.
 // A path tracer's later levels hold ever fewer of its slots: kGroupSlots8.
-// Whole frames: 1280 x 720 (921k) 4.19 ms, dynamic 4.83; 320 x 240 x 16
-// samples (1.23M) 5.41 against 5.82.
+// Whole frames against the persistent kernel: 1280 x 720 (922k) 4.19 and 4.83
+// ms, 320 x 240 x 16 samples (1.23M) 5.41 and 5.82.
 // Up to kAppendSlots of them the group trace takes the later levels' records in
 // the order they were appended: a group's lanes share one ray, so sorting
 // buys less than its six launches a level.  Whole frames of 5 levels, us,
 // sorted / not: hall 480 x 270 1045 / 906, 640 x 480 1770 / 1665, 1120 x 630
 // (706k) 3340 / 3285, 1280 x 720 (922k) 4170 / 4180, 480 x 270 x 8 samples
-// (1.04M) 4555 / 4610; the 8,192-triangle scene 650 / 506, 1070 / 931, 2010 /
+// (1.04M) 4555 / 4610; a hall of 74,068 650 / 506, 1070 / 931, 2010 /
 // 1878, 2525 / 2395, 2890 / 2660; 2 slots per pixel for 8 samples of 480 x 270
 // 7030 / 6060 and 4995 / 3460.
 constexpr uint32_t kAppendSlots = 7u << 17;

@@ -251,7 +251,8 @@ typedef struct {
  * hiprt_tracer_name returns the canonical name. */
 enum {
     HIPRT_TRACER_WHILE_WHILE = 0,                        /* plain: one ray per lane, grid = batch */
-    HIPRT_TRACER_PERSISTENT_WHILE_WHILE = 1,             /* persistent waves, one atomic per fetch */
+    HIPRT_TRACER_PERSISTENT_WHILE_WHILE = 1,             /* persistent waves, one atomic per fetch; one binary
+                                                            tree: the plain kernel, the same bits sooner */
     HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE = 2, /* + leaf postponement */
     HIPRT_TRACER_DYNAMIC_WHILE_WHILE = 3,                /* + leaf postponement + dynamic refill;
                                                             2 and 3 may return either triangle
