@@ -21,8 +21,10 @@
 //     after each leaf phase (8.3 M random rays 5635 us, when it leaves 6496).
 //     70 VGPRs (any-hit), 71 (closest) and 74 (closest, table).
 //
-// Bound: VALU issue (99% of it on 8.3 M bounce rays, at 32% of the lanes) and
-// L1 (1.05 line accesses a clock there) at once; on camera rays VALU alone.
+// Bound, 8.3 M hall rays: L1 lines on incoherent rays (bounce: 1.06 line
+// accesses a clock, address units 98% busy, VALU 89% at 44% of the lanes;
+// trace_persistent's kernel: VALU 99% at 32%), VALU issue on camera rays (all
+// of it at 64% of the lanes, before 54%).
 // Measured, trace_persistent's kernel (its fastest stack configuration for
 // single scenes) -> this one, us.  Closest hit, dynamic tracer, hall camera /
 // bounce / random rays: 921 k 733 -> 657, 1036 -> 956, 1026 -> 950; 2.07 M
