@@ -52,6 +52,7 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
     std::map<std::pair<int, int>, std::vector<rt::dev::batch_desc>> groups;
     std::map<std::pair<int, int>, uint64_t> totals;
     std::map<std::pair<int, int>, int> need;
+    std::map<std::pair<int, int>, bool> lds;   // every tree's nodes within the LDS-stack kernel's reach
     for (uint32_t k = 0; k < n_entries; ++k) {
         const hiprt_batch_entry &e = entries[k];
         if (!e.scene) return fail(HIPRT_ERR_ARG, "entry " + std::to_string(k) + ": null scene");
@@ -75,6 +76,8 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
         totals[key] += e.n;
         if (totals[key] > 0xF0000000ull) return fail(HIPRT_ERR_ARG, "too many rays in one batch");
         need[key] = std::max(need[key], e.scene->stack_need);
+        if (!lds.count(key)) lds[key] = true;
+        if (e.scene->stack_need > 0 && e.scene->lds_need() == 0) lds[key] = false;
         groups[key].push_back(d);
     }
     if (!ctx) return ok();
@@ -99,7 +102,9 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
         const bool own_kernel = opts && (opts->blocks > 0 || opts->spill_limit > 0);
         const uint32_t rays8 = !any && cfg.speculative ? rt::dev::kGroupRays8Spec : rt::dev::kGroupRays8;
         const int lanes = own_kernel ? 0 : rt::dev::group_lanes(bvh, need[g.first], (uint32_t)totals[g.first], rays8);
-        if (!lanes) HIP_TRY(hiprt_detail::attach_spill(st, s, fmt, any != 0, true, need[g.first], cfg, opts ? opts->spill_limit : 0));
+        if (!lanes)
+            HIP_TRY(hiprt_detail::attach_spill(st, s, fmt, any != 0, true, need[g.first],
+                                               lds[g.first] ? need[g.first] : 0, cfg, opts ? opts->spill_limit : 0));
         auto *dst = reinterpret_cast<rt::dev::batch_desc *>(static_cast<char *>(table.p) + off);
         HIP_TRY(hipMemcpy(dst, g.second.data(), g.second.size() * sizeof(rt::dev::batch_desc), hipMemcpyHostToDevice));
         if (lanes)
@@ -200,7 +205,7 @@ int hiprt_autotune(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, const hip
                                                                                      : std::vector<int>{40};
             hiprt_tracer_opts base{40, 0, nullptr, stack, 1, 0, 0};
             rt::dev::persistent_cfg pc = cfg_for(tracer, &base);
-            pc.need = layouts[f]->stack_need;
+            pc.need = layouts[f]->lds_need();
             int full = 0;
             HIP_TRY(rt::dev::persistent_grid(layouts[f]->desc, any != 0, pc, &full));
             for (int thr : thresholds)

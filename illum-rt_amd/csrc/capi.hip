@@ -49,9 +49,9 @@ rt::scene_desc desc_for(const hiprt_scene_s *sc, bool alpha) {
 }
 
 hipError_t attach_spill(hiprt_stream_state *st, hipStream_t s, const rt::scene_desc &d, bool any, bool multi,
-                        int need, rt::dev::persistent_cfg &cfg, int spill_limit) {
+                        int need, int lds_need, rt::dev::persistent_cfg &cfg, int spill_limit) {
     cfg.spill = nullptr;
-    cfg.need = spill_limit > 0 ? 0 : need;
+    cfg.need = spill_limit > 0 ? 0 : lds_need;
     const bool lds = rt::dev::dynamic_fits(d.bvh, any, multi, cfg);
     if (lds && (any || multi)) return hipSuccess;   // the whole stack is in LDS
     cfg.spill_cap = lds ? rt::dev::dynamic_spill_entries(need) : rt::dev::persistent_spill_entries(d.bvh, cfg.stack, need);
@@ -933,7 +933,7 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     } else {
         hiprt_stream_state *st = sc->ctx->state(stream);
         if (!st) return fail(HIPRT_ERR_HIP, "cannot allocate the stream's work counters");
-        HIP_TRY(hiprt_detail::attach_spill(st, s, desc, any, false, need, cfg, opts ? opts->spill_limit : 0));
+        HIP_TRY(hiprt_detail::attach_spill(st, s, desc, any, false, need, sc->lds_need(), cfg, opts ? opts->spill_limit : 0));
         counter = st->counter.as<uint32_t>();
     }
     HIP_TRY(rt::dev::launch_trace_persistent(desc, r, h, occluded, n, nullptr, counter, any, cfg, s));

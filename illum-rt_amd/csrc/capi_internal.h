@@ -118,6 +118,9 @@ struct hiprt_scene_s {
     float light_integral = 0.0f;
     hiprt_detail::dbuf refit_ranges, refit_boxes;   // leaf slots below each child; box tree over the slots (refit)
     rt::scene_desc desc{};
+    // Stack need as the LDS-stack kernel takes it: 0, which keeps that kernel
+    // out, for trees of more nodes than its 32-bit byte offsets reach.
+    int lds_need() const { return n_nodes > rt::dev::kDynamicNodes ? 0 : stack_need; }
 };
 
 namespace hiprt_detail {
@@ -144,8 +147,9 @@ rt::scene_desc desc_for(const hiprt_scene_s *sc, bool alpha);
 // configuration's VGPR and LDS entries hold them): the stream state's
 // buffer, grown once the stream's earlier launches, which may still use the
 // old one, have finished.  `multi` selects the descriptor-table kernel;
+// lds_need (hiprt_scene_s::lds_need) 0 keeps the LDS-stack kernel out;
 // spill_limit > 0 caps the entries per lane (hiprt_tracer_opts::spill_limit).
 hipError_t attach_spill(hiprt_stream_state *st, hipStream_t s, const rt::scene_desc &d, bool any, bool multi,
-                        int need, rt::dev::persistent_cfg &cfg, int spill_limit = 0);
+                        int need, int lds_need, rt::dev::persistent_cfg &cfg, int spill_limit = 0);
 
 } // namespace hiprt_detail

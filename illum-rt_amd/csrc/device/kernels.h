@@ -108,6 +108,10 @@ hipError_t launch_trace_persistent(const scene_desc &sc, const ray_soa &rays, co
 // call these.  dynamic_spill_entries: cfg.spill_cap of a closest-hit launch of
 // one scene (0 when the stack fits); the others need no column.
 constexpr int kDynamicStackNeed = 32;
+// Nodes whose byte offsets fit the kernel's 32-bit offset register (a 64-bit
+// address per lane costs two registers); the caller sets cfg.need to 0 for
+// larger trees, which only an upload whose leaves share slots can have.
+constexpr uint32_t kDynamicNodes = 1u << 26;
 bool dynamic_fits(int bvh, bool any, bool multi, const persistent_cfg &cfg);
 uint32_t dynamic_spill_entries(int need);
 hipError_t dynamic_grid(int tri, bool any, bool multi, const persistent_cfg &cfg, int *blocks);
