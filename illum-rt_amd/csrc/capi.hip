@@ -864,6 +864,38 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
         if (need > rt::dev::kPlainStackCap - 1)
             return fail(HIPRT_ERR_UNSUPPORTED, "BVH deeper than the traversal stack (" + std::to_string(need) + " entries)");
     }
+    rt::dev::persistent_cfg cfg{};
+    cfg.speculative = tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
+    cfg.refill = tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
+    cfg.refill_thr = (opts && opts->refill_threshold > 0) ? opts->refill_threshold : 40;
+    if (cfg.refill_thr > 64) cfg.refill_thr = 64;
+    cfg.blocks = (opts && opts->blocks > 0) ? opts->blocks : 0;
+    cfg.stats = opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats) : nullptr;
+    cfg.stack = stack;
+    cfg.chunks = (opts && opts->work_chunks == 1) ? 1 : 8;
+    cfg.park = (opts && opts->park_leaves > 0 && opts->park_leaves < rt::dev::kParkClosest) ? opts->park_leaves
+                                                                                          : rt::dev::kParkClosest;
+    // The allocation-free trace refuses a tree, stack configuration and grid
+    // whose spill column its scratch cannot hold, at every batch size: a
+    // caller learns it from the first small batch, not from the first large
+    // one.
+    if (noalloc && tracer != HIPRT_TRACER_WHILE_WHILE) {
+        cfg.spill_cap = rt::dev::persistent_spill_entries(desc.bvh, cfg.stack, need);
+        if (opts && opts->spill_limit > 0 && cfg.spill_cap > (uint32_t)opts->spill_limit)
+            cfg.spill_cap = (uint32_t)opts->spill_limit;
+        if (cfg.spill_cap) {
+            int blocks = 0;
+            HIP_TRY(rt::dev::persistent_grid(desc, any, cfg, &blocks));
+            const size_t bytes = rt::dev::persistent_spill_bytes(blocks, cfg.spill_cap);
+            if (bytes > kNoAllocSpillBytes)
+                return fail(HIPRT_ERR_UNSUPPORTED,
+                            "the traversal stack's spill column needs " + std::to_string(bytes) + " bytes (" +
+                                std::to_string(blocks) + " blocks x " + std::to_string(cfg.spill_cap) +
+                                " entries per lane); the allocation-free trace holds " +
+                                std::to_string(kNoAllocSpillBytes) +
+                                ": use fewer blocks, a stack configuration with more entries, or hiprt_trace_closest");
+        }
+    }
     // Small batches: several lanes per ray, whichever tracer was asked for
     // (its hits are the plain tracer's, which every tracer returns up to
     // ties).  A caller that counts fetches, sets the grid or bounds the spill
@@ -885,25 +917,13 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     // column that a scratch limit has to judge keeps its own kernel.
     const bool plain = tracer == HIPRT_TRACER_WHILE_WHILE ||
                        (tracer == HIPRT_TRACER_PERSISTENT_WHILE_WHILE && !own_kernel && desc.bvh == rt::BVH2 &&
-                        need < rt::dev::kPlainStackCap &&
-                        (!noalloc || rt::dev::persistent_spill_entries(desc.bvh, stack, need) == 0));
+                        need < rt::dev::kPlainStackCap && (!noalloc || cfg.spill_cap == 0));
     if (plain) {
         HIP_TRY(rt::dev::launch_trace_plain(desc, r, h, occluded, n, any, need, s,
                                             opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats)
                                                  : nullptr));
         return ok();
     }
-    rt::dev::persistent_cfg cfg{};
-    cfg.speculative = tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
-    cfg.refill = tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
-    cfg.refill_thr = (opts && opts->refill_threshold > 0) ? opts->refill_threshold : 40;
-    if (cfg.refill_thr > 64) cfg.refill_thr = 64;
-    cfg.blocks = (opts && opts->blocks > 0) ? opts->blocks : 0;
-    cfg.stats = opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats) : nullptr;
-    cfg.stack = stack;
-    cfg.chunks = (opts && opts->work_chunks == 1) ? 1 : 8;
-    cfg.park = (opts && opts->park_leaves > 0 && opts->park_leaves < rt::dev::kParkClosest) ? opts->park_leaves
-                                                                                          : rt::dev::kParkClosest;
     uint32_t *counter = nullptr;
     if (noalloc) {
         char *base = nullptr;
@@ -913,20 +933,7 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
         }
         if (!base) return fail(HIPRT_ERR_HIP, "the device's scratch is not set up");
         counter = reinterpret_cast<uint32_t *>(base);
-        cfg.spill_cap = rt::dev::persistent_spill_entries(desc.bvh, cfg.stack, need);
-        if (opts && opts->spill_limit > 0 && cfg.spill_cap > (uint32_t)opts->spill_limit)
-            cfg.spill_cap = (uint32_t)opts->spill_limit;
         if (cfg.spill_cap) {
-            int blocks = 0;
-            HIP_TRY(rt::dev::persistent_grid(desc, any, cfg, &blocks));
-            const size_t bytes = rt::dev::persistent_spill_bytes(blocks, cfg.spill_cap);
-            if (bytes > kNoAllocSpillBytes)
-                return fail(HIPRT_ERR_UNSUPPORTED,
-                            "the traversal stack's spill column needs " + std::to_string(bytes) + " bytes (" +
-                                std::to_string(blocks) + " blocks x " + std::to_string(cfg.spill_cap) +
-                                " entries per lane); the allocation-free trace holds " +
-                                std::to_string(kNoAllocSpillBytes) +
-                                ": use fewer blocks, a stack configuration with more entries, or hiprt_trace_closest");
             cfg.spill = reinterpret_cast<int32_t *>(base + rt::dev::kCounterBytes);
             cfg.spill_bytes = kNoAllocSpillBytes;
         }
