@@ -52,8 +52,22 @@ hipError_t attach_spill(hiprt_stream_state *st, hipStream_t s, const rt::scene_d
                         int need, int lds_need, rt::dev::persistent_cfg &cfg, int spill_limit) {
     cfg.spill = nullptr;
     cfg.need = spill_limit > 0 ? 0 : lds_need;
-    const bool lds = rt::dev::dynamic_fits(d.bvh, any, multi, cfg);
+    bool lds = rt::dev::dynamic_fits(d.bvh, any, multi, cfg);
     if (lds && (any || multi)) return hipSuccess;   // the whole stack is in LDS
+    // A graph keeps the column's address while the stream's buffer may be
+    // replaced by a larger one, and a capturing stream can neither wait nor
+    // allocate: a captured launch takes the kernel whose stack configuration
+    // needs a column for deeper trees only.  (The null stream is never
+    // captured.)
+    if (lds && s && rt::dev::dynamic_spill_entries(need) > 0) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        hipError_t e = hipStreamIsCapturing(s, &capture);
+        if (e != hipSuccess) return e;
+        if (capture != hipStreamCaptureStatusNone) {
+            cfg.need = 0;
+            lds = false;
+        }
+    }
     cfg.spill_cap = lds ? rt::dev::dynamic_spill_entries(need) : rt::dev::persistent_spill_entries(d.bvh, cfg.stack, need);
     if (spill_limit > 0 && cfg.spill_cap > (uint32_t)spill_limit) cfg.spill_cap = (uint32_t)spill_limit;
     cfg.spill_bytes = 0;
