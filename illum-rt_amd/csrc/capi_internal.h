@@ -105,6 +105,7 @@ struct hiprt_scene_s {
     rt::flat_scene host;                         // host copy of the uploaded layout (a scene built on the
                                                  // device: its scalars only, see host_nodes)
     uint32_t n_nodes = 0, n_slots = 0;
+    rt::node2 root{};                            // inner node 0 as a device build wrote it
     hiprt_detail::dbuf arena;                    // one allocation behind the buffers below (device builds)
     hiprt_detail::dbuf nodes, tris, slot_ids;    // traversal data
     hiprt_detail::dbuf tri_geo, mats;            // shading data (scenes committed from a host scene)

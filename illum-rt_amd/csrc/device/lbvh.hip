@@ -120,8 +120,8 @@ __global__ __launch_bounds__(kBlock) void k_tri_boxes(lbvh_in in, lbvh_out out, 
             geo[k] = make_float4(x, y, z, k ? 0.0f : __uint_as_float(m));
             box_grow(b, x, y, z);
         }
-        if (bad) atomicAdd(out.counts + 2, 1u);
-        if (m >= in.n_mats) atomicAdd(out.counts + 4, 1u);
+        if (bad) atomicAdd(out.result->counts + 2, 1u);
+        if (m >= in.n_mats) atomicAdd(out.result->counts + 4, 1u);
         tri_box[i] = b;
         box_grow(c, 0.5f * (b.lo[0] + b.hi[0]), 0.5f * (b.lo[1] + b.hi[1]), 0.5f * (b.lo[2] + b.hi[2]));
     }
@@ -343,7 +343,8 @@ __device__ __forceinline__ int32_t child_ref(const tree_view &v, const int32_t *
 }
 
 __global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *rank, const uint32_t *begins,
-                                                 const box6 *boxes, node2 *nodes, int32_t *root_ref, uint32_t *counts) {
+                                                 const box6 *boxes, node2 *nodes, lbvh_result *result) {
+    uint32_t *counts = result->counts;
     const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (i >= v.n - 1) return;
     const int o = v.other[i], first = min(i, o), last = max(i, o), g = v.split[i];
@@ -369,7 +370,11 @@ __global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *ran
     out[1] = make_float4(br.lo[0], br.hi[0], br.lo[1], br.hi[1]);
     out[2] = make_float4(bl.lo[2], bl.hi[2], br.lo[2], br.hi[2]);
     out[3] = make_float4(__int_as_float(l), __int_as_float(r), 0.0f, 0.0f);
-    if (i == 0) *root_ref = 0;
+    if (i == 0) {
+        result->root_ref = 0;
+        float4 *copy = reinterpret_cast<float4 *>(&result->root);
+        for (int k = 0; k < 4; ++k) copy[k] = out[k];
+    }
 }
 
 // ---- 4. records in Morton order and the lower levels of the box tree ----
@@ -394,11 +399,11 @@ __global__ __launch_bounds__(kBoxBlock) void k_records(lbvh_in in, lbvh_out out,
 }
 
 // Trees of at most max_leaf triangles (including one triangle): the root is a leaf.
-__global__ void k_root_leaf(uint32_t n, int32_t *root_ref, uint32_t *counts) {
+__global__ void k_root_leaf(uint32_t n, lbvh_result *result) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        *root_ref = n ? make_leaf_ref(0u, n) : kInvalidRef;
-        counts[0] = 0;
-        counts[1] = 0;
+        result->root_ref = n ? make_leaf_ref(0u, n) : kInvalidRef;
+        result->counts[0] = 0;
+        result->counts[1] = 0;
     }
 }
 
@@ -417,11 +422,12 @@ size_t lbvh_scratch_bytes(uint32_t n_tris) {
 
 hipError_t launch_lbvh(const lbvh_in &in, const lbvh_out &out, void *scratch, hipStream_t s) {
     const uint32_t n = in.n_tris;
-    hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, s, out.counts);
+    uint32_t *counts = out.result->counts;   // an address, not read here
+    hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, s, counts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (n == 0) {
-        hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, s, 0u, out.root_ref, out.counts);
+        hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, s, 0u, out.result);
         return hipGetLastError();
     }
     const scratch_map sm = map_scratch(n, sort_storage(n));
@@ -446,7 +452,7 @@ hipError_t launch_lbvh(const lbvh_in &in, const lbvh_out &out, void *scratch, hi
     hipLaunchKernelGGL(k_records, dim3((n + kBoxBlock - 1) / kBoxBlock), dim3(kBoxBlock), 0, s, in, out, vals1, boxes);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (n <= (uint32_t)in.max_leaf) {
-        hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, s, n, out.root_ref, out.counts);
+        hipLaunchKernelGGL(k_root_leaf, dim3(1), dim3(64), 0, s, n, out.result);
         return hipGetLastError();
     }
     if ((e = launch_box_tree_top(boxes, n, s)) != hipSuccess) return e;
@@ -461,12 +467,11 @@ hipError_t launch_lbvh(const lbvh_in &in, const lbvh_out &out, void *scratch, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_chains, dim3(n_tiles), dim3(kScanTile), 0, s, v, rank, chains, tiles);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanTile), 0, s, tiles, n_tiles, out.counts);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kScanTile), 0, s, tiles, n_tiles, counts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_number, dim3(n_tiles), dim3(kScanTile), 0, s, chains, tiles, n, begins, out.counts);
+    hipLaunchKernelGGL(k_number, dim3(n_tiles), dim3(kScanTile), 0, s, chains, tiles, n, begins, counts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_emit, grid_for(n - 1), dim3(kBlock), 0, s, v, rank, begins, boxes, out.nodes, out.root_ref,
-                       out.counts);
+    hipLaunchKernelGGL(k_emit, grid_for(n - 1), dim3(kBlock), 0, s, v, rank, begins, boxes, out.nodes, out.result);
     return hipGetLastError();
 }
 

@@ -26,10 +26,16 @@ struct lbvh_out {
     uint32_t *slot_ids;      // n_tris
     float *tri_geo;          // 12 floats per triangle: A.xyz + material bits, B.xyz, C.xyz (w words 0)
     uint32_t *tri_vidx;      // copy of the 3 vertex indices per triangle
-    int32_t *root_ref;       // device int32: root inner node 0, or the leaf reference of a one-leaf tree
-    uint32_t *counts;        // device uint32[5]: emitted inner nodes, depth (inner nodes on the longest path),
-                             // triangles with a bad vertex index, nodes that failed the layout check,
-                             // triangles with a bad material id
+    struct lbvh_result *result;   // device memory
+};
+
+// What the host reads back of a build.
+struct lbvh_result {
+    int32_t root_ref;        // root inner node 0, or the leaf reference of a one-leaf tree
+    uint32_t counts[5];      // emitted inner nodes, depth (inner nodes on the longest path), triangles with a bad
+                             // vertex index, nodes that failed the layout check, triangles with a bad material id
+    uint32_t pad[2];
+    node2 root;              // copy of inner node 0 (trees that have one)
 };
 
 // Scratch the build needs, in bytes, for n_tris triangles.

@@ -50,7 +50,7 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
         return e;
     };
     HIP_TRY(need(scratch, scratch_bytes));
-    HIP_TRY(need(st->build_result, 64));
+    HIP_TRY(need(st->build_result, sizeof(rt::dev::lbvh_result)));
     std::vector<float> mats(8 * (n_materials ? n_materials : 1), 0.0f);
     if (n_materials) std::memcpy(mats.data(), materials, 32ull * n_materials);
     // one allocation for the scene: each hipMalloc of this size takes 20-30 us
@@ -70,26 +70,21 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
             at += align(q.bytes);
         }
     }
-    int32_t *d_root = st->build_result.as<int32_t>();
-    uint32_t *d_counts = reinterpret_cast<uint32_t *>(d_root + 1);
-
+    auto *d_result = st->build_result.as<rt::dev::lbvh_result>();
     rt::dev::lbvh_in in{d_positions, d_indices, d_materials, n_vert, n, n_materials ? n_materials : 1, max_leaf, tri_format};
     rt::dev::lbvh_out o{sc->nodes.as<rt::node2>(), sc->tris.as<rt::tri_rec>(), sc->slot_ids.as<uint32_t>(),
-                        sc->tri_geo.as<float>(),   sc->tri_vidx.as<uint32_t>(), d_root, d_counts};
+                        sc->tri_geo.as<float>(),   sc->tri_vidx.as<uint32_t>(), d_result};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (device_ms) {
         HIP_TRY(hipEventCreate(&e0));
         HIP_TRY(hipEventCreate(&e1));
         HIP_TRY(hipEventRecord(e0, s));
     }
-    struct {
-        int32_t root;
-        uint32_t counts[5];
-    } res{};
+    rt::dev::lbvh_result res{};
     hipError_t le = rt::dev::launch_lbvh(in, o, scratch.p, s);
     if (device_ms && le == hipSuccess) le = hipEventRecord(e1, s);
     if (le == hipSuccess) le = hipMemcpyAsync(sc->mats.p, mats.data(), mats.size() * 4, hipMemcpyHostToDevice, s);
-    if (le == hipSuccess) le = hipMemcpyAsync(&res, d_root, sizeof res, hipMemcpyDeviceToHost, s);
+    if (le == hipSuccess) le = hipMemcpyAsync(&res, d_result, sizeof res, hipMemcpyDeviceToHost, s);
     // (waits also after a failed launch: the buffers must be idle when freed)
     hipError_t we = hipStreamSynchronize(s);
     if (le == hipSuccess) le = we;
@@ -111,7 +106,8 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     rt::flat_scene &h = sc->host;
     h.bvh_kind = rt::BVH2;
     h.tri_kind = tri_format;
-    h.root_ref = res.root;
+    h.root_ref = res.root_ref;
+    sc->root = res.root;
     h.depth = counts[1];
     hiprt_detail::set_desc(sc.get(), counts[1]);
     sc->n_nodes = counts[0];

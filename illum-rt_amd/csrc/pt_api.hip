@@ -32,7 +32,7 @@ namespace {
 
 // Sort grid over the scene box: the union of the root's child boxes (a
 // one-leaf or empty tree sorts by the direction's cell or octant only).
-hipError_t grid_of(const hiprt_scene_s *sc, rt::dev::sort_grid *out) {
+rt::dev::sort_grid grid_of(const hiprt_scene_s *sc) {
     const rt::flat_scene &h = sc->host;
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     auto grow = [&](float xl, float xh, float yl, float yh, float zl, float zh) {
@@ -44,13 +44,10 @@ hipError_t grid_of(const hiprt_scene_s *sc, rt::dev::sort_grid *out) {
         hi[2] = std::max(hi[2], zh);
     };
     if (h.root_ref >= 0 && h.bvh_kind == rt::BVH2 && (uint32_t)h.root_ref < sc->n_nodes) {
-        rt::node2 r;
-        if (h.nodes2.empty()) {   // built on the device
-            hipError_t e = hipMemcpy(&r, sc->nodes.as<const rt::node2>() + h.root_ref, sizeof r, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) return e;
-        } else {
-            r = h.nodes2[h.root_ref];
-        }
+        // (built on the device: the host keeps the root as it was built; either
+        // kind of scene is sorted by its box from before any refit, which no
+        // work still queued on a stream can change)
+        const rt::node2 &r = h.nodes2.empty() ? sc->root : h.nodes2[h.root_ref];
         grow(r.lxlo, r.lxhi, r.lylo, r.lyhi, r.lzlo, r.lzhi);
         grow(r.rxlo, r.rxhi, r.rylo, r.ryhi, r.rzlo, r.rzhi);
     } else if (h.root_ref >= 0 && h.bvh_kind == rt::BVH4 && (size_t)h.root_ref < h.nodes4.size()) {
@@ -66,8 +63,7 @@ hipError_t grid_of(const hiprt_scene_s *sc, rt::dev::sort_grid *out) {
         g.scale[a] = ok_axis ? (float)(1u << rt::dev::kSortCellBits) / ext : 0.0f;
         if (!std::isfinite(g.scale[a])) g.scale[a] = 0.0f;
     }
-    *out = g;
-    return hipSuccess;
+    return g;
 }
 
 // Shading data of a committed scene for the device steps.
@@ -727,7 +723,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
         HIP_TRY(p->perm.alloc(4ull * n));
         HIP_TRY(p->sort_counts.alloc(4ull * 256 * rt::dev::radix_tiles(n)));
         HIP_TRY(p->sort_totals.alloc(4ull * 256));
-        HIP_TRY(grid_of(sc, &p->grid));
+        p->grid = grid_of(sc);
     }
     if (p->batched) {
         p->pcfg.need = sc->lds_need();
