@@ -886,6 +886,7 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     cfg.blocks = (opts && opts->blocks > 0) ? opts->blocks : 0;
     cfg.stats = opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats) : nullptr;
     cfg.stack = stack;
+    cfg.rays = n;
     cfg.chunks = (opts && opts->work_chunks == 1) ? 1 : 8;
     cfg.park = (opts && opts->park_leaves > 0 && opts->park_leaves < rt::dev::kParkClosest) ? opts->park_leaves
                                                                                           : rt::dev::kParkClosest;

@@ -88,6 +88,7 @@ struct persistent_cfg {
     uint32_t spill_cap = 0;
     size_t spill_bytes = 0;
     int need = 0;         // the trees' stack need; 0: trace_persistent.hip's kernels (see dynamic_fits)
+    uint32_t rays = 0xffffffffu;   // rays of the launch, or as many as it can have (sizes the grid of one scene)
 };
 
 // `counter` points to kCounterBytes of device memory (cleared by the launch);

@@ -303,9 +303,26 @@ constexpr uint32_t kSentinels = 2;
 // least alike, and more wavefronts evict each other's nodes (3 x 1.1 M rays
 // of 250 k triangles: 6 blocks 2745 us, 5 2620, 4 2395; 24 x 200 k of 5 k
 // 1580, 1560, 1615).  Any-hit keeps all: camera rays, 8.3 M, 3012 us with 6
-// blocks, 3451 with 4.
+// blocks, 3451 with 4.  (Random any-hit rays are the exception: 8.3 M of the
+// hall 6428 us with 7 blocks, 6043 with 5, 2.07 M 1843 and 1774; camera rays pay
+// for it, 2810 and 2920.)
+//
+// One scene and few rays: a grid of 7 blocks per CU is 459 k lanes, so up to a
+// million rays most lanes take one or two, the rays of a wavefront are spread
+// over the batch by its end, and every further block adds its start and its
+// round of empty work counters.  Closest hit, dynamic tracer, 5 / 6 / 7 blocks,
+// camera and bounce rays: 500 triangles, 640 k rays 116 / 123 / 133 and 130 / 146 /
+// 169; 2.07 M 182 / 188 / 195 and 206 / 208 / 216; 8,192 triangles, 640 k 193 /
+// 206 / 220 and 232 / 243 / 265; 2.07 M 312 / 310 / 303 and 364 / 369 / 364;
+// 130,000, 800 k 353 / 366 / 373 and 386 / 415 / 429; hall, 1 M 696 / 661 / 658
+// and 950 / 938 / 972, 1.3 M 802 / 766 / 750 and 1116 / 1106 / 1117.
+inline int few_rays_blocks(int need, uint32_t rays) {
+    if (rays <= 1u << 20) return need <= 14 ? 5 : 6;
+    return rays <= 1u << 21 && need <= 12 ? 5 : 8;
+}
+
 template <int TRI, bool ANY, bool MULTI>
-hipError_t grid_of(uint32_t entries, bool refill, int *blocks) {
+hipError_t grid_of(uint32_t entries, const persistent_cfg &cfg, int *blocks) {
     static int cached[64][kDynamicStackNeed + kSentinels + 1] = {};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -321,7 +338,8 @@ hipError_t grid_of(uint32_t entries, bool refill, int *blocks) {
         if (per_cu < 1) per_cu = 1;
         cached[dev][entries] = per_cu;
     }
-    if (MULTI && !ANY && refill && per_cu > 4) per_cu = 4;
+    if (MULTI && !ANY && cfg.refill && per_cu > 4) per_cu = 4;
+    if (!MULTI) per_cu = min(per_cu, few_rays_blocks(cfg.need, cfg.rays));
     *blocks = cus * per_cu;
     return hipSuccess;
 }
@@ -330,7 +348,7 @@ template <int TRI, bool ANY, bool MULTI>
 hipError_t launch_one(const dynamic_args &a, const persistent_cfg &cfg, hipStream_t s, int *grid_out) {
     int blocks = cfg.blocks;
     if (blocks <= 0) {
-        hipError_t e = grid_of<TRI, ANY, MULTI>(a.entries, cfg.refill, &blocks);
+        hipError_t e = grid_of<TRI, ANY, MULTI>(a.entries, cfg, &blocks);
         if (e != hipSuccess) return e;
     }
     if (grid_out) {

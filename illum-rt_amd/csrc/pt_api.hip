@@ -727,6 +727,7 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
     }
     if (p->batched) {
         p->pcfg.need = sc->lds_need();
+        p->pcfg.rays = n;
         // Resolve the persistent grid size outside the capture, then record
         // the frame once.  The graph never clears the accumulator: frame 0
         // after a reset is rendered eagerly with clear_radiance set.
