@@ -12,6 +12,7 @@
 #include "core/raygen.h"
 #include "device/kernels.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -494,7 +495,8 @@ std::string check_layout(rt::flat_scene &f, uint32_t &stack_need) {
 typedef float float_x4 __attribute__((vector_size(16)));
 typedef int int_x4 __attribute__((vector_size(16)));
 
-static void check_boxes(const rt::flat_scene &h, bool &nan_free, bool &nested) {
+// (also sums half the surface of a binary tree's inner and leaf boxes)
+static void check_boxes(const rt::flat_scene &h, bool &nan_free, bool &nested, double &inner, double &leaf) {
     const bool binary = h.bvh_kind == rt::BVH2;
     const size_t n = binary ? h.nodes2.size() : h.nodes4.size();
     const float_x4 *f = binary ? reinterpret_cast<const float_x4 *>(h.nodes2.data())
@@ -512,9 +514,17 @@ static void check_boxes(const rt::flat_scene &h, bool &nan_free, bool &nested) {
             const float_x4 lo = __builtin_shufflevector(l, r, 0, 2, 4, 6), hi = __builtin_shufflevector(l, r, 1, 3, 5, 7);
             out |= ~(lo <= -hi) | ~(lz <= -__builtin_shufflevector(lz, lz, 1, 0, 1, 0)) |
                    ~(rz <= -__builtin_shufflevector(rz, rz, 1, 0, 1, 0));
+            const float_x4 e = -(lo + hi);   // extents x, y of the left and the right box
+            const float ez_l = -(lz[0] + lz[1]), ez_r = -(rz[0] + rz[1]);
+            const float area[2] = {e[0] * e[1] + (e[0] + e[1]) * ez_l, e[2] * e[3] + (e[2] + e[3]) * ez_r};
             for (int k = 0; k < 2; ++k) {
                 const int32_t ref = k ? h.nodes2[i].ref_r : h.nodes2[i].ref_l;
-                if (rt::ref_is_leaf(ref)) continue;
+                const float half = area[k];
+                if (rt::ref_is_leaf(ref)) {
+                    leaf += half;
+                    continue;
+                }
+                inner += half;
                 const float_x4 *c = f + 4 * (size_t)ref;
                 const float_x4 xy = k ? r : l, zz = __builtin_shufflevector(k ? rz : lz, z, 0, 1, 0, 1);
                 out |= ~(c[0] * sign >= xy) | ~(c[1] * sign >= xy) | ~(c[2] * sign >= zz);
@@ -538,9 +548,23 @@ void set_desc(hiprt_scene_s *s, uint32_t stack_need) {
     s->n_nodes = (uint32_t)(h.bvh_kind == rt::BVH2 ? h.nodes2.size() : h.nodes4.size());
     s->n_slots = (uint32_t)h.tris.size();
     bool nan_free = true, nested = false;
-    check_boxes(h, nan_free, nested);
+    double inner = 0, leaf = 0;
+    check_boxes(h, nan_free, nested, inner, leaf);
+    if (h.bvh_kind == rt::BVH2 && h.root_ref >= 0 && (size_t)h.root_ref < h.nodes2.size())
+        s->group_rays = group_rays_of(inner, leaf, h.nodes2[h.root_ref]);
     s->desc.nan_free = nan_free ? 1 : 0;
     s->desc.nested = nested ? 1 : 0;
+}
+
+uint32_t group_rays_of(double inner, double leaf, const rt::node2 &r) {
+    const double x = std::fmax(r.lxhi, r.rxhi) - std::fmin(r.lxlo, r.rxlo),
+                 y = std::fmax(r.lyhi, r.ryhi) - std::fmin(r.lylo, r.rylo),
+                 z = std::fmax(r.lzhi, r.rzhi) - std::fmin(r.lzlo, r.rzlo);
+    const double root = x * y + (x + y) * z, sl = leaf / root, sn = 1.0 + inner / root;
+    const double rays = 570000.0 * sl * sl * (sn - 3.0) / (sn * sn);
+    // boxes that are no boxes (empty, infinite, inverted) say nothing
+    if (!(root > 0.0 && inner >= 0.0 && leaf > 0.0 && rays < 1e9)) return rt::dev::kGroupRays16;
+    return rays > rt::dev::kGroupRays16 ? (uint32_t)rays : rt::dev::kGroupRays16;
 }
 
 hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
@@ -917,8 +941,9 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     // column gets the kernel those belong to.
     const bool own_kernel = opts && (opts->d_fetch_stats || opts->blocks > 0 || opts->spill_limit > 0);
     const bool postpones = !any && tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
-    const uint32_t rays8 = postpones ? rt::dev::kGroupRays8Spec : rt::dev::kGroupRays8;
-    if (int lanes = own_kernel ? 0 : rt::dev::group_lanes(desc.bvh, need, n, rays8)) {
+    const uint32_t few = postpones ? rt::dev::kGroupRays8Spec : rt::dev::kGroupRays8;
+    const uint64_t tree = any ? sc->group_rays * 8ull / 5 : sc->group_rays;   // any-hit ends sooner: 0.8 of the time
+    if (int lanes = own_kernel ? 0 : rt::dev::group_lanes(desc.bvh, need, n, (uint32_t)std::min<uint64_t>(few, tree))) {
         HIP_TRY(rt::dev::launch_trace_group(desc, r, h, occluded, n, nullptr, any, lanes, need, s));
         return ok();
     }
@@ -928,11 +953,21 @@ int trace_common(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t *oc
     // hit, stack 0 / stack 4 / plain, us: camera 1466 / 1361 / 1181, bounce
     // 2727 / 2280 / 2069, random 2751 / 2350 / 2171; soup 365 / 355 / 255, 488 /
     // 447 / 367, 1363 / 1224 / 1005; 500 triangles 185 / 221 / 102.  Any-hit
-    // likewise (bounce 2545 / 2143 / 2155, else ahead by 5-50%).  A spill
-    // column that a scratch limit has to judge keeps its own kernel.
+    // likewise (bounce 2545 / 2143 / 2155, else ahead by 5-50%).  Behind at 8.3 M:
+    // camera rays of the 74,068-triangle hall against stack 4, closest hit 1373 /
+    // 1490.  A spill column that a scratch limit has to judge keeps its own
+    // kernel.
+    //
+    // Few rays of a light tree, beyond what the group trace serves: the plain
+    // kernel whichever tracer was asked for.  A persistent grid's start and
+    // tail are most of such a launch: closest hit, plain / dynamic / group, us of
+    // camera, bounce, random rays: 500 triangles, 500 k rays 61 / 133 / 79, 90 /
+    // 165 / 61, 172 / 183 / 176; small hall, 640 k 229 / 267 / 324, 320 / 317 / 350,
+    // 306 / 303 / 365; any-hit, 1 M rays of the small hall 264 / 309 / 441, 424 /
+    // 413 / 429, 375 / 392 / 416.
     const bool plain = tracer == HIPRT_TRACER_WHILE_WHILE ||
-                       (tracer == HIPRT_TRACER_PERSISTENT_WHILE_WHILE && !own_kernel && desc.bvh == rt::BVH2 &&
-                        need < rt::dev::kPlainStackCap && (!noalloc || cfg.spill_cap == 0));
+                       ((tracer == HIPRT_TRACER_PERSISTENT_WHILE_WHILE || n <= few) && !own_kernel &&
+                        desc.bvh == rt::BVH2 && need < rt::dev::kPlainStackCap && (!noalloc || cfg.spill_cap == 0));
     if (plain) {
         HIP_TRY(rt::dev::launch_trace_plain(desc, r, h, occluded, n, any, need, s,
                                             opts ? reinterpret_cast<unsigned long long *>(opts->d_fetch_stats)

@@ -106,6 +106,7 @@ struct hiprt_scene_s {
                                                  // device: its scalars only, see host_nodes)
     uint32_t n_nodes = 0, n_slots = 0;
     rt::node2 root{};                            // inner node 0 as a device build wrote it
+    uint32_t group_rays = rt::dev::kGroupRays16; // rays up to which 8 lanes trace one of them (group_rays_of)
     hiprt_detail::dbuf arena;                    // one allocation behind the buffers below (device builds)
     hiprt_detail::dbuf nodes, tris, slot_ids;    // traversal data
     hiprt_detail::dbuf tri_geo, mats;            // shading data (scenes committed from a host scene)
@@ -135,6 +136,27 @@ std::string check_layout(rt::flat_scene &f, uint32_t &stack_need);
 // on the device copies them into `fetched` from device memory).
 hipError_t host_nodes(const hiprt_scene_s *s, std::vector<rt::node2> &fetched, const rt::node2 *&nodes2,
                       const rt::node4 *&nodes4);
+
+// Rays of one binary tree up to which the group trace's 8 lanes per ray are the
+// faster (the launch's own limit applies too): `inner` and `leaf` sum half the
+// surface of its inner nodes' boxes, without the root's, and of its leaves'.
+//
+// Over the root's surface these are the nodes Sn and leaves Sl that a random
+// line meets.  Plain and persistent kernels have a floor, the slowest
+// wavefront, and a slope that leaves set; the group trace pays for nodes and
+// a fixed part per ray and has next to no floor, so it holds on the longer the
+// more of a ray's work is leaves.  570,000 Sl^2 / Sn (1 - 3 / Sn) fits the measured
+// crossings over random triangles and both halls.  Sl, Sn, limit; us of camera
+// and random rays, closest hit, group / plain:
+//   100 triangles     1.9   7.8  155 k  at 200 k 30 / 34, 60 / 54     300 k 41 / 34, 85 / 65
+//   500               3.5  17.3  334 k  at 300 k 54 / 57, 113 / 118   500 k 79 / 61, 176 / 172
+//   2,000             6.3  32.3  631 k  at 500 k 95 / 105, 233 / 256  800 k 145 / 138, 363 / 333
+//   8,192            10.9  58.3  1.11 M at 800 k 174 / 207, 449 / 465  1 M 210 / 283, 550 / 558
+//   74,068 (hall)     6.5  53.7  421 k  at 400 k 216 / 321, 239 / 229  640 k 324 / 229, 365 / 306
+//   262,144 (hall)   17.6   131  1.31 M at 800 k 660 / 661, 765 / 1006  1 M 809 / 900, 943 / 1157
+// A limit on the ray count alone, 1 M, took 481 us for 1 M camera rays of the
+// small hall (plain 352) and 147 us for those of 500 triangles (plain 95).
+uint32_t group_rays_of(double inner, double leaf, const rt::node2 &root);
 
 // Fills the scene descriptor from the device buffers and the host copy.
 void set_desc(hiprt_scene_s *s, uint32_t stack_need);

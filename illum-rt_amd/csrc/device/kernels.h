@@ -139,7 +139,9 @@ hipError_t persistent_grid(const scene_desc &sc, bool any, const persistent_cfg 
 // to fill the chip with one ray per lane.  group_lanes: 16 up to kGroupRays16
 // rays, 8 up to kGroupRays8 (kGroupRays8Spec for the closest hits of the
 // postponing tracers), else 0, and 0 for 4-wide or very deep trees: the plain
-// and persistent kernels serve those.  Hall, us, camera / bounce rays:
+// and persistent kernels serve those.  Callers pass the tree's own limit
+// (hiprt_detail::group_rays_of) where that is lower.  Hall, us, camera / bounce
+// rays:
 //   16 -> 8: 320 x 240 (77k) 124 / 131 against 129 / 139, but 53 / 41 against
 //   43 / 44 in the 8,192-triangle scene.
 //   8 -> 0: 960 x 540 (518k) 504 / 547, plain 576 / 789; 1280 x 720 (922k)

@@ -342,11 +342,16 @@ __device__ __forceinline__ int32_t child_ref(const tree_view &v, const int32_t *
     return (int32_t)(begins[first] + (uint32_t)rank[c]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *rank, const uint32_t *begins,
-                                                 const box6 *boxes, node2 *nodes, lbvh_result *result) {
+__device__ __forceinline__ float half_area(const box6 &b) {
+    const float x = b.hi[0] - b.lo[0], y = b.hi[1] - b.lo[1], z = b.hi[2] - b.lo[2];
+    return x >= 0.0f && y >= 0.0f && z >= 0.0f ? x * y + (x + y) * z : 0.0f;
+}
+
+// Inner node i; area.x and area.y: half the surface of its inner children's
+// boxes and of its leaves'.
+__device__ __forceinline__ void emit_node(const tree_view &v, int i, const int32_t *rank, const uint32_t *begins,
+                                          const box6 *boxes, node2 *nodes, lbvh_result *result, float2 &area) {
     uint32_t *counts = result->counts;
-    const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (i >= v.n - 1) return;
     const int o = v.other[i], first = min(i, o), last = max(i, o), g = v.split[i];
     if (!emitted(v, first, last)) return;
     // what the host checks of an uploaded tree: the node and its inner
@@ -374,6 +379,31 @@ __global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *ran
         result->root_ref = 0;
         float4 *copy = reinterpret_cast<float4 *>(&result->root);
         for (int k = 0; k < 4; ++k) copy[k] = out[k];
+    }
+    const float al = half_area(bl), ar = half_area(br);
+    area.x = (l >= 0 ? al : 0.0f) + (r >= 0 ? ar : 0.0f);
+    area.y = (l >= 0 ? 0.0f : al) + (r >= 0 ? 0.0f : ar);
+}
+
+__global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *rank, const uint32_t *begins,
+                                                 const box6 *boxes, node2 *nodes, lbvh_result *result, float2 *areas) {
+    __shared__ float2 sum[kBlock / 64];
+    const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
+    float2 area = make_float2(0.0f, 0.0f);
+    if (i < v.n - 1) emit_node(v, i, rank, begins, boxes, nodes, result, area);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        area.x += __shfl_down(area.x, off, 64);
+        area.y += __shfl_down(area.y, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) sum[threadIdx.x >> 6] = area;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / 64; ++w) {
+            area.x += sum[w].x;
+            area.y += sum[w].y;
+        }
+        areas[blockIdx.x] = area;
     }
 }
 
@@ -414,6 +444,8 @@ __global__ void k_clear(uint32_t *counts) {
 inline dim3 grid_for(uint32_t n) { return dim3((n + kBlock - 1) / kBlock); }
 
 } // namespace
+
+uint32_t lbvh_area_blocks(uint32_t n_tris) { return n_tris > 1 ? grid_for(n_tris - 1).x : 0u; }
 
 size_t lbvh_scratch_bytes(uint32_t n_tris) {
     if (n_tris == 0) return 256;
@@ -471,7 +503,8 @@ hipError_t launch_lbvh(const lbvh_in &in, const lbvh_out &out, void *scratch, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_number, dim3(n_tiles), dim3(kScanTile), 0, s, chains, tiles, n, begins, counts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_emit, grid_for(n - 1), dim3(kBlock), 0, s, v, rank, begins, boxes, out.nodes, out.result);
+    hipLaunchKernelGGL(k_emit, grid_for(n - 1), dim3(kBlock), 0, s, v, rank, begins, boxes, out.nodes, out.result,
+                       out.areas);
     return hipGetLastError();
 }
 

@@ -27,6 +27,8 @@ struct lbvh_out {
     float *tri_geo;          // 12 floats per triangle: A.xyz + material bits, B.xyz, C.xyz (w words 0)
     uint32_t *tri_vidx;      // copy of the 3 vertex indices per triangle
     struct lbvh_result *result;   // device memory
+    float2 *areas;                // lbvh_area_blocks: sums of half the surface of inner children's boxes and of leaves'
+                                  // (written for trees with inner nodes)
 };
 
 // What the host reads back of a build.
@@ -37,6 +39,8 @@ struct lbvh_result {
     uint32_t pad[2];
     node2 root;              // copy of inner node 0 (trees that have one)
 };
+
+uint32_t lbvh_area_blocks(uint32_t n_tris);
 
 // Scratch the build needs, in bytes, for n_tris triangles.
 size_t lbvh_scratch_bytes(uint32_t n_tris);

@@ -50,7 +50,10 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
         return e;
     };
     HIP_TRY(need(scratch, scratch_bytes));
-    HIP_TRY(need(st->build_result, sizeof(rt::dev::lbvh_result)));
+    const uint32_t n_areas = rt::dev::lbvh_area_blocks(n);
+    const size_t result_bytes = sizeof(rt::dev::lbvh_result) + n_areas * sizeof(float2);
+    HIP_TRY(need(st->build_result, result_bytes));
+    std::vector<char> host_result(result_bytes);
     std::vector<float> mats(8 * (n_materials ? n_materials : 1), 0.0f);
     if (n_materials) std::memcpy(mats.data(), materials, 32ull * n_materials);
     // one allocation for the scene: each hipMalloc of this size takes 20-30 us
@@ -73,18 +76,18 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     auto *d_result = st->build_result.as<rt::dev::lbvh_result>();
     rt::dev::lbvh_in in{d_positions, d_indices, d_materials, n_vert, n, n_materials ? n_materials : 1, max_leaf, tri_format};
     rt::dev::lbvh_out o{sc->nodes.as<rt::node2>(), sc->tris.as<rt::tri_rec>(), sc->slot_ids.as<uint32_t>(),
-                        sc->tri_geo.as<float>(),   sc->tri_vidx.as<uint32_t>(), d_result};
+                        sc->tri_geo.as<float>(),   sc->tri_vidx.as<uint32_t>(), d_result,
+                        reinterpret_cast<float2 *>(d_result + 1)};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (device_ms) {
         HIP_TRY(hipEventCreate(&e0));
         HIP_TRY(hipEventCreate(&e1));
         HIP_TRY(hipEventRecord(e0, s));
     }
-    rt::dev::lbvh_result res{};
     hipError_t le = rt::dev::launch_lbvh(in, o, scratch.p, s);
     if (device_ms && le == hipSuccess) le = hipEventRecord(e1, s);
     if (le == hipSuccess) le = hipMemcpyAsync(sc->mats.p, mats.data(), mats.size() * 4, hipMemcpyHostToDevice, s);
-    if (le == hipSuccess) le = hipMemcpyAsync(&res, d_result, sizeof res, hipMemcpyDeviceToHost, s);
+    if (le == hipSuccess) le = hipMemcpyAsync(host_result.data(), d_result, result_bytes, hipMemcpyDeviceToHost, s);
     // (waits also after a failed launch: the buffers must be idle when freed)
     hipError_t we = hipStreamSynchronize(s);
     if (le == hipSuccess) le = we;
@@ -93,6 +96,7 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     if (e1) (void)hipEventDestroy(e1);
     if (le != hipSuccess) return fail(HIPRT_ERR_HIP, std::string("device BVH build: ") + hipGetErrorString(le));
 
+    const auto &res = *reinterpret_cast<const rt::dev::lbvh_result *>(host_result.data());
     const uint32_t *counts = res.counts;
     if (counts[2]) return fail(HIPRT_ERR_ARG, std::to_string(counts[2]) + " triangles name a vertex past n_vert");
     if (counts[3]) return fail(HIPRT_ERR_HIP, "device BVH build produced a node off the tree");
@@ -112,6 +116,15 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     hiprt_detail::set_desc(sc.get(), counts[1]);
     sc->n_nodes = counts[0];
     sc->n_slots = n;
+    if (counts[0]) {
+        const auto *areas = reinterpret_cast<const float2 *>(host_result.data() + sizeof res);
+        double inner = 0, leaf = 0;
+        for (uint32_t k = 0; k < n_areas; ++k) {
+            inner += areas[k].x;
+            leaf += areas[k].y;
+        }
+        sc->group_rays = hiprt_detail::group_rays_of(inner, leaf, res.root);
+    }
     sc->desc.nan_free = 1;
     sc->desc.nested = 1;   // unions; a subtree of empty boxes holds no triangle to hit
     sc->n_tris = n;

@@ -703,7 +703,11 @@ int hiprt_pt_create(hiprt_scene sc, const float *cam, const hiprt_pt_params *par
     HIP_TRY(hipMemset(p->totals.p, 0, 8ull * (p->pp.max_depth + 1)));
     HIP_TRY(p->frame_seed.alloc(8ull * samples));
     HIP_TRY(p->work.alloc(rt::dev::kCounterBytes));
-    if (params->blocks <= 0) p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n, rt::dev::kGroupSlots8);
+    if (params->blocks <= 0) {
+        const uint64_t tree = (uint64_t)sc->group_rays * 3 / 2;   // as for kGroupSlots8: later levels hold fewer rays
+        p->group = rt::dev::group_lanes(sc->desc.bvh, sc->stack_need, n,
+                                        (uint32_t)std::min<uint64_t>(rt::dev::kGroupSlots8, tree));
+    }
     p->append_order = p->group && n <= rt::dev::kAppendSlots;
     p->pcfg.speculative = p->tracer >= HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE;
     p->pcfg.refill = p->tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
