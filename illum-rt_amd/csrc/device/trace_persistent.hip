@@ -27,9 +27,10 @@
 //     children sorted by entry distance, the nearest entered, the others
 //     pushed farthest first;
 //   * without postponement, a vote that ends the node loop once at most
-//     kNodeLanes lanes still descend (1920 x 1080 rays of the hall,
+//     kNodeLanes lanes still descend (VOTE; 1920 x 1080 rays of the hall,
 //     persistent-while-while, stack 3: camera 1563 -> 1369 us, bounce 3133 ->
-//     2444, random 2911 -> 2480);
+//     2444, random 2911 -> 2480).  Shallow binary trees go without: its ballot
+//     costs each node step more than the few idle lanes (kVoteNeed);
 //   * a descriptor table (MULTI): the rays of many scenes form one index
 //     space; each lane binds the scene of the ray it fetched, so one launch
 //     traces uneven batches of many scenes;
@@ -196,7 +197,7 @@ constexpr int waves_hint(int reg, int lds, int bvh, bool multi) {
     return reg == 0 && lds == 20 && bvh == 2 && !multi ? 8 : 1;
 }
 
-template <int TRI, bool ANY, bool SPEC, bool REFILL, int REG, int LDS, bool COUNT, int BVH, bool MULTI, bool RING>
+template <int TRI, bool ANY, bool SPEC, bool REFILL, int REG, int LDS, bool COUNT, int BVH, bool MULTI, bool RING, bool VOTE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_hint(REG, LDS, BVH, MULTI))))
 void k_trace_persistent(scene_desc sc, ray_soa rays, hit_soa hits, uint8_t *occluded, uint32_t n_static,
                         const uint32_t *count_ptr, uint32_t *counter, int lane_limits, unsigned long long *stats,
@@ -361,7 +362,7 @@ void k_trace_persistent(scene_desc sc, ray_soa rays, hit_soa hits, uint8_t *occl
                         }
                         searching = pc == 0;
                         if (__ballot(searching) == 0) break;
-                    } else if (__popcll(__ballot(cur >= 0 && cur != kInvalidRef)) <= kNodeLanes) {
+                    } else if (VOTE && __popcll(__ballot(cur >= 0 && cur != kInvalidRef)) <= kNodeLanes) {
                         break;
                     }
                 }
@@ -469,7 +470,7 @@ constexpr int lds_for(int bvh, int stk) {
 
 // Blocks of one instantiation that fit the device at once (occupancy x CUs),
 // asked once per device.
-template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK, bool RING>
+template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK, bool RING, bool VOTE>
 hipError_t grid_of(int *blocks) {
     static int cached[64] = {0};
     int dev = 0;
@@ -482,7 +483,8 @@ hipError_t grid_of(int *blocks) {
         if (e != hipSuccess) return e;
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu,
-            k_trace_persistent<TRI, ANY, SPEC, REFILL, reg_for(STK), lds_for(BVH, STK), false, BVH, MULTI, RING>, 256,
+            k_trace_persistent<TRI, ANY, SPEC, REFILL, reg_for(STK), lds_for(BVH, STK), false, BVH, MULTI, RING,
+                               VOTE>, 256,
             0);
         if (e != hipSuccess) return e;
         cached[dev] = cus * (per_cu > 0 ? per_cu : 1);
@@ -514,12 +516,12 @@ inline int lane_limits_of(const persistent_cfg &cfg) {
     return thr | (park << 8);
 }
 
-template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK, bool RING>
+template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK, bool RING, bool VOTE>
 hipError_t launch_ring(const launch_args &a, const persistent_cfg &cfg, hipStream_t stream, bool grid_only,
                        int *grid_out) {
     int blocks = cfg.blocks;
     if (blocks <= 0) {
-        hipError_t e = grid_of<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, RING>(&blocks);
+        hipError_t e = grid_of<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, RING, VOTE>(&blocks);
         if (e != hipSuccess) return e;
     }
     if (grid_out) *grid_out = blocks;
@@ -530,14 +532,14 @@ hipError_t launch_ring(const launch_args &a, const persistent_cfg &cfg, hipStrea
     constexpr int R = reg_for(STK), L = lds_for(BVH, STK);
     if constexpr (!MULTI && RING) {
         if (cfg.stats) {
-            hipLaunchKernelGGL((k_trace_persistent<TRI, ANY, SPEC, REFILL, R, L, true, BVH, MULTI, true>),
+            hipLaunchKernelGGL((k_trace_persistent<TRI, ANY, SPEC, REFILL, R, L, true, BVH, MULTI, true, VOTE>),
                                dim3(blocks), dim3(256), 0, stream, a.sc, a.rays, a.hits, a.occluded, a.n, a.count_ptr,
                                a.counter, lane_limits_of(cfg), cfg.stats, a.table, a.n_desc, chunks_of(cfg.chunks),
                                cfg.spill, cfg.spill_cap, a.gather);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((k_trace_persistent<TRI, ANY, SPEC, REFILL, R, L, false, BVH, MULTI, RING>), dim3(blocks),
+    hipLaunchKernelGGL((k_trace_persistent<TRI, ANY, SPEC, REFILL, R, L, false, BVH, MULTI, RING, VOTE>), dim3(blocks),
                        dim3(256), 0, stream, a.sc, a.rays, a.hits, a.occluded, a.n, a.count_ptr, a.counter,
                        lane_limits_of(cfg), cfg.stats, a.table, a.n_desc, chunks_of(cfg.chunks), cfg.spill, cfg.spill_cap,
                        a.gather);
@@ -547,24 +549,35 @@ hipError_t launch_ring(const launch_args &a, const persistent_cfg &cfg, hipStrea
 // The plain LDS stack runs single-scene launches whose tree fits the
 // configuration; descriptor-table launches, counting launches and trees
 // that spill use the ring.
-template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK>
+template <int TRI, bool ANY, bool SPEC, bool REFILL, int BVH, bool MULTI, int STK, bool VOTE>
 hipError_t launch_variant(const launch_args &a, const persistent_cfg &cfg, hipStream_t stream, bool grid_only,
                           int *grid_out) {
     if constexpr (!MULTI) {
         if (!cfg.stats && cfg.spill_cap == 0)
-            return launch_ring<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, false>(a, cfg, stream, grid_only, grid_out);
+            return launch_ring<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, false, VOTE>(a, cfg, stream, grid_only, grid_out);
     }
-    return launch_ring<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, true>(a, cfg, stream, grid_only, grid_out);
+    return launch_ring<TRI, ANY, SPEC, REFILL, BVH, MULTI, STK, true, VOTE>(a, cfg, stream, grid_only, grid_out);
 }
+
+// Binary trees of more stack entries than this vote.  Tables, closest hit,
+// random rays, without / with the vote: 32 x 60 k rays of 500 triangles 738 / 787
+// us, of 1,000 890 / 930, 24 x 60 k of 5,000 1024 / 1043, of 30,000 (16 entries)
+// 1480 / 1480; 3 x 200 k camera rays of the hall (22 entries) 1050 / 866, 4 x 500 k
+// random rays of the 74,068-triangle hall (20) 990 / 952.
+constexpr int kVoteNeed = 16;
 
 template <int TRI, bool ANY, int BVH, bool MULTI, int STK>
 hipError_t dispatch_flags(const launch_args &a, const persistent_cfg &cfg, hipStream_t s, bool grid_only, int *g) {
     if (cfg.speculative) {
-        if (cfg.refill) return launch_variant<TRI, ANY, true, true, BVH, MULTI, STK>(a, cfg, s, grid_only, g);
-        return launch_variant<TRI, ANY, true, false, BVH, MULTI, STK>(a, cfg, s, grid_only, g);
+        if (cfg.refill) return launch_variant<TRI, ANY, true, true, BVH, MULTI, STK, false>(a, cfg, s, grid_only, g);
+        return launch_variant<TRI, ANY, true, false, BVH, MULTI, STK, false>(a, cfg, s, grid_only, g);
     }
-    if (cfg.refill) return launch_variant<TRI, ANY, false, true, BVH, MULTI, STK>(a, cfg, s, grid_only, g);
-    return launch_variant<TRI, ANY, false, false, BVH, MULTI, STK>(a, cfg, s, grid_only, g);
+    // (only the postponing tracer refills)
+    if constexpr (BVH == 2) {
+        if (cfg.need > 0 && cfg.need <= kVoteNeed)
+            return launch_variant<TRI, ANY, false, false, BVH, MULTI, STK, false>(a, cfg, s, grid_only, g);
+    }
+    return launch_variant<TRI, ANY, false, false, BVH, MULTI, STK, true>(a, cfg, s, grid_only, g);
 }
 
 template <int TRI, bool ANY, int BVH, bool MULTI>
