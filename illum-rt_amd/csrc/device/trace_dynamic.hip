@@ -315,9 +315,10 @@ constexpr uint32_t kSentinels = 2;
 // 169; 2.07 M 182 / 188 / 195 and 206 / 208 / 216; 8,192 triangles, 640 k 193 /
 // 206 / 220 and 232 / 243 / 265; 2.07 M 312 / 310 / 303 and 364 / 369 / 364;
 // 130,000, 800 k 353 / 366 / 373 and 386 / 415 / 429; hall, 1 M 696 / 661 / 658
-// and 950 / 938 / 972, 1.3 M 802 / 766 / 750 and 1116 / 1106 / 1117.
-inline int few_rays_blocks(int need, uint32_t rays) {
-    if (rays <= 1u << 20) return need <= 14 ? 5 : 6;
+// and 950 / 938 / 972, 1.3 M 802 / 766 / 750 and 1116 / 1106 / 1117.  (Without
+// refill the hall's trees take them all: bounce rays, 1 M, 1039 / 1010 with 6 / 7.)
+inline int few_rays_blocks(int need, uint32_t rays, bool refill) {
+    if (rays <= 1u << 20) return need <= 14 ? 5 : (refill || need <= 19 ? 6 : 8);
     return rays <= 1u << 21 && need <= 12 ? 5 : 8;
 }
 
@@ -339,7 +340,7 @@ hipError_t grid_of(uint32_t entries, const persistent_cfg &cfg, int *blocks) {
         cached[dev][entries] = per_cu;
     }
     if (MULTI && !ANY && cfg.refill && per_cu > 4) per_cu = 4;
-    if (!MULTI) per_cu = min(per_cu, few_rays_blocks(cfg.need, cfg.rays));
+    if (!MULTI) per_cu = min(per_cu, few_rays_blocks(cfg.need, cfg.rays, cfg.refill));
     *blocks = cus * per_cu;
     return hipSuccess;
 }

@@ -487,6 +487,10 @@ hipError_t grid_of(int *blocks) {
                                VOTE>, 256,
             0);
         if (e != hipSuccess) return e;
+        // A seventh block of the postponing 4-wide kernels with 20 LDS words
+        // costs 20 k rays of 500 triangles 122 -> 131 us and of the hall up to 3%,
+        // and 2.07 M rays gain nothing from it.
+        if (BVH == 4 && SPEC && !REFILL && STK == 4 && per_cu > 6) per_cu = 6;
         cached[dev] = cus * (per_cu > 0 ? per_cu : 1);
     }
     *blocks = cached[dev];
