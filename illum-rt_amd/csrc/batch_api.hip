@@ -155,9 +155,11 @@ int hiprt_autotune(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, const hip
     }
     // A persistent grid holds ~300k lanes on MI355X: a batch much smaller than
     // that times tail latency, not throughput, and ranks configurations
-    // wrongly.  Small samples are therefore tiled up to kMinTuneRays rays;
-    // results are checked on the first n (the sample itself).
-    constexpr uint32_t kMinTuneRays = 1u << 20;
+    // wrongly; up to kGroupRays8 rays the launch's rules by batch size choose
+    // the kernel, not the configuration.  Small samples are therefore tiled up
+    // to kMinTuneRays rays; results are checked on the first n (the sample
+    // itself).
+    constexpr uint32_t kMinTuneRays = rt::dev::kGroupRays8 + 1;
     const uint32_t reps = n >= kMinTuneRays ? 1u : (kMinTuneRays + n - 1) / n;
     const uint64_t nt64 = (uint64_t)n * reps;
     if (nt64 > 0xF0000000ull) {
@@ -208,19 +210,26 @@ int hiprt_autotune(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, const hip
     hiprt_tune_result best{};
     float best_ms = 1e30f;
     int count = 0;
+    // Candidates run on the default grid (blocks 0), which the result keeps:
+    // a caller's own grid would rule out the kernels for small batches.
     for (int f = 0; f < 2; ++f)
     for (int stack = 0; stack < rt::dev::kStackConfigs; ++stack) {
         for (int tracer = HIPRT_TRACER_PERSISTENT_WHILE_WHILE; tracer < HIPRT_TRACER_COUNT; ++tracer) {
             std::vector<int> thresholds = tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE ? std::vector<int>{24, 40, 56}
                                                                                      : std::vector<int>{40};
+            // what one kernel serves is timed once: the postponing kernel with
+            // its stack in LDS has no stack configurations, the plain kernel
+            // behind persistent-while-while no work counters either
             hiprt_tracer_opts base{40, 0, nullptr, stack, 1, 0, 0};
             rt::dev::persistent_cfg pc = cfg_for(tracer, &base);
             pc.need = layouts[f]->lds_need();
-            int full = 0;
-            HIP_TRY(rt::dev::persistent_grid(layouts[f]->desc, any != 0, pc, &full));
+            const bool plain = f == rt::BVH2 && tracer == HIPRT_TRACER_PERSISTENT_WHILE_WHILE &&
+                               layouts[f]->stack_need < rt::dev::kPlainStackCap;
+            if (stack > 0 && (plain || rt::dev::dynamic_fits(f, any != 0, false, pc))) continue;
             for (int thr : thresholds)
                 for (int chunks : {1, 8}) {
-                    hiprt_tracer_opts o{thr, full, nullptr, stack, chunks, 0, 0};
+                    if (plain && chunks == 1) continue;
+                    hiprt_tracer_opts o{thr, 0, nullptr, stack, chunks, 0, 0};
                     if (int st = trace(layouts[f], tracer, &o, &h, nt)) return st;
                     float ms = 1e30f;
                     for (int rep = 0; rep < 2; ++rep) {

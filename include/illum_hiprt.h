@@ -352,18 +352,20 @@ int hiprt_trace_batch(const hiprt_batch_entry *entries, uint32_t n_entries, int3
  * Times candidate configurations on a sample of a scene's rays -- tracer
  * variant (persistent / speculative / dynamic), refill threshold, stack
  * configuration, work chunks and BVH layout (binary vs collapsed 4-wide), on
- * the occupancy-derived grid, then the parked-leaf limit of the winner -- and
- * returns the fastest.  A sample of fewer
- * than 2^20 rays is tiled up to that size before timing: a batch smaller than
- * the lanes a persistent grid holds (~300k) measures tail latency and ranks
- * configurations wrongly.  Every candidate's hits on the sample are compared
+ * the default grid, then the parked-leaf limit of the winner -- and
+ * returns the fastest; options that a candidate's kernel does not read are
+ * not varied.  A sample of at most 2^20 rays is tiled beyond that size before
+ * timing: a batch smaller than the lanes a persistent grid holds (~300k)
+ * measures tail latency and ranks configurations wrongly, and smaller
+ * batches over binary trees take other kernels whatever is asked for
+ * (hiprt_tracer_opts).  Every candidate's hits on the sample are compared
  * with the plain kernel's; a candidate that differs other than at equal t is
  * rejected.  Results never depend on the choice.  The scene is committed in
  * the chosen layout into *tuned (caller destroys it). */
 typedef struct {
     int32_t tracer;
     int32_t refill_threshold;
-    int32_t blocks;
+    int32_t blocks;        /* 0: the default grid */
     int32_t bvh_format;
     float mrays_per_s;     /* measured on the sample */
     int32_t candidates;    /* configurations timed */
