@@ -846,18 +846,25 @@ int hiprt_pt_autotune(hiprt_scene bvh2_scene, hiprt_scene bvh4_scene, const floa
     };
     // 1. tracer x layout x stack configuration, one sample
     for (int tracer : {HIPRT_TRACER_DYNAMIC_WHILE_WHILE, HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE}) {
+        // (the postponing kernel with its stack in LDS has no stack configurations)
+        const bool one_stack = bvh2_scene->lds_need() > 0;
         for (int stack : {0, 3, 4})
-            if (int st = consider(HIPRT_BVH2, tracer, stack, 1, rt::dev::kParkClosest)) return st;
+            if (stack == 0 || !one_stack)
+                if (int st = consider(HIPRT_BVH2, tracer, stack, 1, rt::dev::kParkClosest)) return st;
         if (bvh4_scene)
             for (int stack : {0, 3})
                 if (int st = consider(HIPRT_BVH4, tracer, stack, 1, rt::dev::kParkClosest)) return st;
     }
-    // 2. samples in flight for the winner and for the binary tree with stack 4
+    // 2. samples in flight for the winner, and for the binary tree with the
+    // other tracer (with the same one, when the winner is 4-wide): refill and
+    // samples in flight both fill idle lanes
     const hiprt_pt_tune_result one = best;
+    const int other = one.bvh_format != HIPRT_BVH2                      ? one.tracer
+                      : one.tracer == HIPRT_TRACER_DYNAMIC_WHILE_WHILE ? HIPRT_TRACER_PERSISTENT_SPECULATIVE_WHILE_WHILE
+                                                                       : HIPRT_TRACER_DYNAMIC_WHILE_WHILE;
     for (int s = 2; s <= max_s; s *= 2) {
         if (int st = consider(one.bvh_format, one.tracer, one.stack_config, s, rt::dev::kParkClosest)) return st;
-        if (!(one.bvh_format == HIPRT_BVH2 && one.stack_config == 4))
-            if (int st = consider(HIPRT_BVH2, one.tracer, 4, s, rt::dev::kParkClosest)) return st;
+        if (int st = consider(HIPRT_BVH2, other, 0, s, rt::dev::kParkClosest)) return st;
     }
     // 3. parked leaves
     const hiprt_pt_tune_result win = best;

@@ -557,10 +557,9 @@ int hiprt_pt_render(hiprt_pt pt, uint32_t frame, void *stream);
  * samples and park fields are ignored) with candidate configurations and
  * returns the one that traces the most rays per second:
  *   1. tracer (speculative, dynamic) x layout (bvh2_scene; bvh4_scene when not
- *      NULL) x stack configuration (0 and 3; 4 on the binary tree), one
- *      sample per pixel;
+ *      NULL, with stack configurations 0 and 3), one sample per pixel;
  *   2. samples in flight 2, 4, ... up to max_samples for the winner of 1 and
- *      for the binary tree with stack configuration 4;
+ *      for the binary tree with the other tracer;
  *   3. parked leaves 1..3 for the winner.
  * Each candidate renders one warm-up and `trial_frames` (0: 2) timed frames
  * on its own path tracer.  Images do not depend on the choice.  Synchronous. */

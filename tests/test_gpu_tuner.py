@@ -36,3 +36,24 @@ def test_tuned_options_keep_the_default_grid(torch_cuda, hip_ctx, any_hit):
     assert torch.equal(got["t"], want["t"]) and torch.equal(occ, occ_want)
     tuned.close()
     ds.close()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_frame_tuner_leaves_out_equal_candidates(torch_cuda, hip_ctx, wide):
+    """Two samples at most: one candidate per tracer on the binary tree, two per
+    tracer on the 4-wide one, two with two samples in flight, three limits of
+    parked leaves."""
+    sc = hiprt.HostScene.generate(2)
+    cam = sc.cam.copy()
+    cam[10], cam[11] = 96, 54
+    bvh = hiprt.Bvh(sc)
+    ds = hiprt.DeviceScene(hip_ctx, sc, bvh)
+    ds4 = hiprt.DeviceScene(hip_ctx, sc, bvh, hiprt.BVH4) if wide else None
+    print(f"case: frame tuner, 96 x 54, 4-wide tree {wide}", flush=True)
+    kw, info = hiprt.pt_autotune(ds, ds4, cam, max_samples=2)
+    assert info["candidates"] == (2 + 4 * wide) + 2 + 3
+    if info["layout"] == "bvh2":
+        assert kw["stack_config"] == 0
+    for x in (ds, ds4):
+        if x is not None:
+            x.close()
