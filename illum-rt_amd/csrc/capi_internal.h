@@ -85,16 +85,17 @@ struct hiprt_stream_state {
     hiprt_detail::dbuf batch_table;   // descriptor table of the last batched trace on the stream
     hiprt_detail::dbuf spill;         // stack spill buffer of the persistent kernels (grown on demand)
     hiprt_detail::dbuf adjoint;       // sort scratch of the adjoint's vertex accumulation (grown on demand)
-    // device BVH builds: their scratch (bounded, kept between builds) and result words; one
-    // build at a time, which waits for its own work
-    std::mutex build_lock;
-    hiprt_detail::dbuf build_scratch, build_result;
 };
 
 struct hiprt_context_s {
     int device = 0;
     std::mutex lock;                  // guards `streams`
     std::map<void *, std::unique_ptr<hiprt_stream_state>> streams;
+    // Device BVH builds: scratch and result words kept for the next build on
+    // any stream (a build waits for its own work, so they are idle between
+    // builds).  A build that finds them in use allocates its own.
+    std::mutex build_lock;
+    hiprt_detail::dbuf build_scratch, build_result;
     // The state of `stream` (created on first use, counters zeroed); null on
     // allocation failure.
     hiprt_stream_state *state(void *stream);

@@ -15,7 +15,7 @@ using hiprt_detail::ok;
 
 namespace {
 // Build scratch up to this size (about 1.5 million triangles) stays with the
-// stream's state for the next build; more is returned after the call.
+// context for the next build; more is returned after the call.
 constexpr size_t kKeptScratchBytes = size_t(256) << 20;
 } // namespace
 
@@ -36,13 +36,11 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     if (!sc) return fail(HIPRT_ERR_ARG, "out of host memory");
     sc->ctx = ctx;
     const uint32_t n = n_tris, m = n > 1 ? n - 1 : 1, n1 = n ? n : 1;
-    hiprt_stream_state *st = ctx->state(stream);
-    if (!st) return fail(HIPRT_ERR_HIP, "cannot allocate the stream's work counters");
-    std::lock_guard<std::mutex> g(st->build_lock);
     const size_t scratch_bytes = rt::dev::lbvh_scratch_bytes(n);
-    const bool kept = scratch_bytes <= kKeptScratchBytes;
-    dbuf own;
-    dbuf &scratch = kept ? st->build_scratch : own;
+    dbuf own, own_result;   // (freed after the lock: theirs is not shared)
+    std::unique_lock<std::mutex> mine(ctx->build_lock, std::try_to_lock);
+    dbuf &scratch = mine.owns_lock() && scratch_bytes <= kKeptScratchBytes ? ctx->build_scratch : own;
+    dbuf &result = mine.owns_lock() ? ctx->build_result : own_result;
     auto need = [](dbuf &b, size_t bytes) {   // (the last build that used it has ended)
         if (b.bytes >= bytes) return hipSuccess;
         hipError_t e = b.alloc(bytes);
@@ -52,7 +50,7 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
     HIP_TRY(need(scratch, scratch_bytes));
     const uint32_t n_areas = rt::dev::lbvh_area_blocks(n);
     const size_t result_bytes = sizeof(rt::dev::lbvh_result) + n_areas * sizeof(float2);
-    HIP_TRY(need(st->build_result, result_bytes));
+    HIP_TRY(need(result, result_bytes));
     std::vector<char> host_result(result_bytes);
     std::vector<float> mats(8 * (n_materials ? n_materials : 1), 0.0f);
     if (n_materials) std::memcpy(mats.data(), materials, 32ull * n_materials);
@@ -73,7 +71,7 @@ int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_ve
             at += align(q.bytes);
         }
     }
-    auto *d_result = st->build_result.as<rt::dev::lbvh_result>();
+    auto *d_result = result.as<rt::dev::lbvh_result>();
     rt::dev::lbvh_in in{d_positions, d_indices, d_materials, n_vert, n, n_materials ? n_materials : 1, max_leaf, tri_format};
     rt::dev::lbvh_out o{sc->nodes.as<rt::node2>(), sc->tris.as<rt::tri_rec>(), sc->slot_ids.as<uint32_t>(),
                         sc->tri_geo.as<float>(),   sc->tri_vidx.as<uint32_t>(), d_result,

@@ -198,7 +198,8 @@ int hiprt_scene_commit(hiprt_context ctx, hiprt_host_scene s, hiprt_bvh b, int32
  * hits agree with brute force up to equal-t ties and grazing hits.
  * *device_ms (optional) receives the build kernels' time on `stream`; the
  * call returns after the scene is ready; the tree is checked and stays on the
- * device. */
+ * device.  The context keeps up to 256 MiB of scratch for the next build, until
+ * hiprt_destroy; a build that overlaps another one allocates its own. */
 int hiprt_scene_build(hiprt_context ctx, const float *d_positions, uint32_t n_vert, const uint32_t *d_indices,
                       uint32_t n_tris, const uint32_t *d_materials, const float *materials, uint32_t n_materials,
                       int32_t max_leaf, int32_t tri_format, hiprt_scene *out, float *device_ms, void *stream);
