@@ -20,7 +20,8 @@
 //      walks; an exclusive scan of the chains' lengths gives the numbers, the
 //      difference to the scan of the chains that end at a position the number
 //      of nodes above each leaf, so the depth;
-//   7. nodes written in that order, each child's box a range of the box tree.
+//   7. nodes written in that order, each child's box a range of the box tree;
+//      the surfaces of inner and leaf boxes, summed per block, go to the host.
 //
 // What bounds it is the latency of its launches (20 of them the sort's) and
 // of short dependent loads; no step waits on another wavefront.  The hall's
@@ -49,6 +50,7 @@ namespace dev {
 namespace {
 
 constexpr int kBlock = 256;
+constexpr uint32_t kEmitBlock = 1024;   // few area sums to read back
 constexpr uint32_t kMortonBits = 21;
 constexpr uint32_t kScanTile = 1024;   // positions per block of the numbering scan
 
@@ -385,10 +387,10 @@ __device__ __forceinline__ void emit_node(const tree_view &v, int i, const int32
     area.y = (l >= 0 ? 0.0f : al) + (r >= 0 ? 0.0f : ar);
 }
 
-__global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *rank, const uint32_t *begins,
+__global__ __launch_bounds__(kEmitBlock) void k_emit(tree_view v, const int32_t *rank, const uint32_t *begins,
                                                  const box6 *boxes, node2 *nodes, lbvh_result *result, float2 *areas) {
-    __shared__ float2 sum[kBlock / 64];
-    const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
+    __shared__ float2 sum[kEmitBlock / 64];
+    const int i = (int)(blockIdx.x * kEmitBlock + threadIdx.x);
     float2 area = make_float2(0.0f, 0.0f);
     if (i < v.n - 1) emit_node(v, i, rank, begins, boxes, nodes, result, area);
 #pragma unroll
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(kBlock) void k_emit(tree_view v, const int32_t *ran
     if ((threadIdx.x & 63u) == 0) sum[threadIdx.x >> 6] = area;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < kBlock / 64; ++w) {
+        for (int w = 1; w < kEmitBlock / 64; ++w) {
             area.x += sum[w].x;
             area.y += sum[w].y;
         }
@@ -445,7 +447,7 @@ inline dim3 grid_for(uint32_t n) { return dim3((n + kBlock - 1) / kBlock); }
 
 } // namespace
 
-uint32_t lbvh_area_blocks(uint32_t n_tris) { return n_tris > 1 ? grid_for(n_tris - 1).x : 0u; }
+uint32_t lbvh_area_blocks(uint32_t n_tris) { return n_tris > 1 ? (n_tris - 1 + kEmitBlock - 1) / kEmitBlock : 0u; }
 
 size_t lbvh_scratch_bytes(uint32_t n_tris) {
     if (n_tris == 0) return 256;
@@ -503,7 +505,7 @@ hipError_t launch_lbvh(const lbvh_in &in, const lbvh_out &out, void *scratch, hi
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_number, dim3(n_tiles), dim3(kScanTile), 0, s, chains, tiles, n, begins, counts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_emit, grid_for(n - 1), dim3(kBlock), 0, s, v, rank, begins, boxes, out.nodes, out.result,
+    hipLaunchKernelGGL(k_emit, dim3(lbvh_area_blocks(n)), dim3(kEmitBlock), 0, s, v, rank, begins, boxes, out.nodes, out.result,
                        out.areas);
     return hipGetLastError();
 }
