@@ -95,7 +95,7 @@ def kernel_name(kw, ds, binary):
     ring = "true" if ds.stack_need > reg + lds else "false"
     if spec == "true" and binary and ds.stack_need > 0:   # the stack in LDS, whatever the configuration
         return f"k_trace_dynamic<0, false, false> ({tracer}, binary tree)"
-    vote = "true" if spec == "false" and not (binary and ds.stack_need <= 16) else "false"
+    vote = "true" if spec == "false" and not (binary and ds.stack_need <= 12) else "false"
     return (f"k_trace_persistent<0, false, {spec}, {refill}, {reg}, {lds}, false, {2 if binary else 4}, false, "
             f"{ring}, {vote}> ({tracer}, stack {kw.get('stack_config', 0)}, {'binary' if binary else '4-wide'} tree)")
 

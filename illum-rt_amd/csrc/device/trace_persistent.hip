@@ -564,11 +564,11 @@ hipError_t launch_variant(const launch_args &a, const persistent_cfg &cfg, hipSt
 }
 
 // Binary trees of more stack entries than this vote.  Tables, closest hit,
-// random rays, without / with the vote: 32 x 60 k rays of 500 triangles 738 / 787
-// us, of 1,000 890 / 930, 24 x 60 k of 5,000 1024 / 1043, of 30,000 (16 entries)
-// 1480 / 1480; 3 x 200 k camera rays of the hall (22 entries) 1050 / 866, 4 x 500 k
-// random rays of the 74,068-triangle hall (20) 990 / 952.
-constexpr int kVoteNeed = 16;
+// random rays, stack 0, without / with the vote: 32 x 60 k rays of 500 triangles
+// (9 entries) 738 / 787 us, of 1,000 890 / 930, 24 x 60 k of 5,000 (14) 1024 / 1043
+// (stack 4 975 / 921), of 30,000 (16) 1480 / 1480; 3 x 200 k camera rays of the hall
+// (22) 1050 / 866, 4 x 500 k random rays of the 74,068-triangle hall (20) 990 / 952.
+constexpr int kVoteNeed = 12;
 
 template <int TRI, bool ANY, int BVH, bool MULTI, int STK>
 hipError_t dispatch_flags(const launch_args &a, const persistent_cfg &cfg, hipStream_t s, bool grid_only, int *g) {
