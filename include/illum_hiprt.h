@@ -223,8 +223,10 @@ int hiprt_scene_download(hiprt_scene sc, void *nodes, void *tri_records, uint32_
  * of boxes over the leaf slots (three launches).  Leaf boxes bound whole triangles.  The device
  * counterpart of rebuilding on every commit (rt/cuda/base.cpp:88-117) when
  * only vertices move -- scene-view transforms (rt/cuda/preprocessing.cpp:41-72)
- * or gradient steps on vertices.  Needs a scene from hiprt_scene_commit;
- * stream-ordered, no host synchronisation. */
+ * or gradient steps on vertices.  Needs a scene from hiprt_scene_commit or
+ * hiprt_scene_build; stream-ordered, no host synchronisation after a scene's
+ * first refit, which prepares on the host with blocking copies (of a
+ * device-built scene also the nodes back). */
 int hiprt_scene_refit(hiprt_scene sc, const float *d_positions, void *stream);
 int hiprt_scene_destroy(hiprt_scene sc);
 /* Most traversal-stack entries any ray can need in this tree (the persistent
@@ -250,6 +252,13 @@ typedef struct {
  * persistent-while-while, "speculative-while-while" ->
  * persistent-speculative-while-while (each also with "-alpha");
  * hiprt_tracer_name returns the canonical name. */
+/* A tracer names a traversal, not always a kernel.  Batches over binary trees
+ * of up to 1 M rays (655,360 closest-hit rays of tracers 2 and 3; fewer over
+ * trees that a ray leaves quickly) are traced with 16 or 8 lanes per ray,
+ * then, up to those numbers, with one ray per lane, whichever tracer and
+ * options were asked for: the hits are those of HIPRT_TRACER_WHILE_WHILE.  A
+ * caller that sets blocks, d_fetch_stats or spill_limit gets the tracer's own
+ * kernel at every size. */
 enum {
     HIPRT_TRACER_WHILE_WHILE = 0,                        /* plain: one ray per lane, grid = batch */
     HIPRT_TRACER_PERSISTENT_WHILE_WHILE = 1,             /* persistent waves, one atomic per fetch; one binary
@@ -272,10 +281,12 @@ enum {
 int hiprt_tracer_id(const char *name);
 const char *hiprt_tracer_name(int tracer);
 
-/* Tunables for the persistent tracers (zero = default). */
+/* Tunables for the persistent tracers (zero = default).  Batches that another
+ * kernel serves (above) read none but blocks, d_fetch_stats and spill_limit. */
 typedef struct {
     int32_t refill_threshold; /* refill when fewer lanes of 64 are active (default 40) */
-    int32_t blocks;           /* grid size (default: occupancy x CU count) */
+    int32_t blocks;           /* grid size (default: up to occupancy x CU count, fewer for few rays);
+                                 selects the tracer's own kernel */
     uint64_t *d_fetch_stats;  /* non-NULL: run the counting variant, which adds the inner
                                  nodes it fetches to [0] and the triangle records it
                                  tests to [1] (device uint64[2]) */
@@ -286,8 +297,9 @@ typedef struct {
                                  to a global column per lane.  Speculative launches over
                                  binary trees hold their stack in LDS whatever the
                                  configuration, unless they count fetches, bound the
-                                 spill column or must not allocate (any-hit and batches:
-                                 or the tree needs more than 32 entries) */
+                                 spill column or must not allocate, and closest hits
+                                 under stream capture (any-hit and batches: or the tree
+                                 needs more than 32 entries) */
     int32_t work_chunks;      /* 1 = one work counter; 8 (and 0, the default) = one
                                  contiguous chunk of the rays per XCD, blocks start on
                                  their own XCD's chunk (fetch atomics spread over 8
@@ -323,7 +335,8 @@ int hiprt_trace_any(hiprt_scene sc, const hiprt_rays *rays, uint32_t n, uint8_t 
  * whose spill column (grid blocks x 256 lanes x spill entries per lane x 4 B,
  * entries = the tree's stack need minus the stack configuration's VGPR + LDS
  * entries) exceeds 16 MiB is refused with HIPRT_ERR_UNSUPPORTED before any
- * launch.  Every call on one device shares that scratch: calls that overlap
+ * launch, also for batches so small that their kernel has no column.  Every
+ * call on one device shares that scratch: calls that overlap
  * in time on one device (concurrent streams, threads) race and must be
  * serialized by the caller; consecutive calls on one stream are fine (the
  * counters are cleared by a kernel at each launch). */
@@ -498,8 +511,9 @@ int hiprt_integrate_light_sample(hiprt_scene sc, const hiprt_rays *cam_rays, con
  *                device, the whole frame captured once in a hipGraph.
  * In the batched schedule the queue of every bounce is, by default
  * (ray_order = 0), sorted by direction octant and origin cell (a 16^3 grid
- * over the scene box) so that wavefronts trace neighbouring rays; small frames,
- * which several lanes per ray trace, are not sorted.  1 keeps the order the
+ * over the scene box) so that wavefronts trace neighbouring rays; small frames
+ * over binary trees, which several lanes per ray trace unless blocks is set,
+ * are not sorted up to 917,504 paths.  1 keeps the order the
  * shading step appends them in.  Paths keep their own random
  * streams, so the image does not depend on the order.  samples > 1 traces
  * that many samples per pixel in one frame graph -- render call k traces the
